@@ -162,8 +162,9 @@ int t2_sweeper_create(t2_sweeper **out, int device,
                       int64_t n_groups, const double *sigma_t,
                       const double *sigma_s, int precision, int gauss);
 /* Environment: T2_NO_GRAPH=1 makes the level engine launch its per-step
- * kernels directly instead of replaying a captured hipGraph (a debugging
- * aid; results are identical). */
+ * kernels directly, whatever the problem, instead of replaying a captured
+ * hipGraph or sweeping in one launch (a debugging aid; results are
+ * identical). */
 int t2_sweeper_destroy(t2_sweeper *s);
 int t2_sweeper_info(const t2_sweeper *s, t2_info *info);
 
@@ -230,7 +231,10 @@ int t2_set_priority(t2_sweeper *s, int intra_angle_p, int inter_angle_p,
 
 /* Sweep engine (GraphTraverser::traverse, src/GraphTraverser.cc:467-759):
  *   T2_ENGINE_LEVELS  one kernel launch per schedule step, the whole sweep
- *                     captured once in a hipGraph and replayed (default);
+ *                     captured once in a hipGraph and replayed (default); with
+ *                     the launch and schedule knobs at their defaults, small
+ *                     and deep problems run in one launch instead, a block
+ *                     sweeping an angle through its levels;
  *   T2_ENGINE_QUEUE   one persistent launch: blocks take chunks of items in
  *                     schedule order from a device ticket counter, each item
  *                     waits on its atomic pending-upwind counter, solves, and

@@ -1,0 +1,66 @@
+"""The level engine's one-block-per-angle form (live values in LDS slots)
+against its step launches (T2_NO_GRAPH), bit for bit, at the sizes where the
+form's rounds, slots and group chunks change."""
+import numpy as np
+import pytest
+
+from tycho2_amd import mesh as meshmod
+from tycho2_amd.quadrature import product_quadrature
+from tycho2_amd.sweeper import FP32, FP64, SweeperHIP
+
+pytestmark = pytest.mark.gpu
+
+
+def handle(n, sn, ng, precision, sigma="both", seed=5):
+    sm = meshmod.kuhn_cube(n, 0.15, seed=seed)
+    omega, wt = product_quadrature(sn)
+    rng = np.random.default_rng(seed)
+    cell = rng.uniform(0.5, 2.0, (sm.n_cells, 1))
+    group = 1.0 + 0.1 * np.arange(ng)[None, :]
+    st = np.broadcast_to({"cell": cell, "group": group,
+                          "both": cell * group}[sigma], (sm.n_cells, ng))
+    s = SweeperHIP(sm, meshmod.tycho_connectivity(sm), omega, wt, ng, st,
+                   0.8 * st, precision)
+    s.set_source_isotropic(rng.uniform(0.0, 1.0, (sm.n_cells, 4, ng)))
+    return s
+
+
+def states(s, precision):
+    """psi after sweeps with an isotropic source, psi and phi after three
+    source-iteration steps, and a refined solve's (FP32: the angle-dependent
+    source in flux precision, swept in place)."""
+    out = []
+    for _ in range(3):
+        s.sweep_step()
+    out += [s.psi(), s.phi()]
+    src = np.random.default_rng(9).uniform(0.0, 1.0, out[0].shape)
+    if s.info()["n_lagged"] == 0 or precision == FP64:
+        out.append(s.sweep(np.zeros_like(src), src).copy())
+    if precision == FP32:
+        s.solve_refined(100, 1e-5, 1e-4, 20)
+        out += [s.psi(), s.phi()]
+    return out
+
+
+@pytest.mark.parametrize("n,sn,ng,sigma", [
+    (1, 2, 1, "cell"),       # six cells: every level a part of one round
+    (2, 4, 2, "group"),
+    (5, 4, 1, "both"),       # one group: contiguous rows
+    (6, 6, 1, "cell"),       # angles at 45 degrees: lagged faces
+    (5, 6, 4, "both"),       # ... with group chunks
+    (7, 8, 8, "group"),      # eight groups a block
+    (6, 4, 16, "both"),      # several chunks of groups
+    (3, 8, 64, "cell"),      # most groups
+    (12, 8, 4, "both"),      # levels of several rounds
+])
+@pytest.mark.parametrize("precision", [FP64, FP32])
+def test_equals_step_launches(n, sn, ng, sigma, precision, monkeypatch):
+    print(f"angle form n={n} sn={sn} ng={ng} {sigma} {precision}", flush=True)
+    with handle(n, sn, ng, precision, sigma) as s:
+        got = states(s, precision)
+    monkeypatch.setenv("T2_NO_GRAPH", "1")
+    with handle(n, sn, ng, precision, sigma) as s:
+        ref = states(s, precision)
+    for a, b in zip(got, ref):
+        assert np.isfinite(a).all()
+        assert np.array_equal(a, b)

@@ -92,6 +92,13 @@ struct t2_sweeper {
     int64_t *d_lag_key = nullptr;
     int32_t *d_lag_up = nullptr;
     void *d_lag_buf = nullptr;
+    // one-block-per-angle form of the level sets (angle_gc 0: not built)
+    int angle_gc = 0, angle_block = 0;
+    int64_t angle_slots = 0, angle_lag = 0, n_rounds = 0;
+    t2::SlotItem *d_slot_items = nullptr;
+    t2::AngleRound *d_rounds = nullptr;
+    int32_t *d_angles = nullptr;     // round_off [na + 1], order [na],
+                                     // lag_off [na + 1]
     // fluxes and sources
     void *d_psi = nullptr;           // T [na][nc][4][G]
     void *d_src = nullptr;           // T [nc][4][G]
@@ -283,6 +290,16 @@ int ensure_side_streams(t2_sweeper *s, int64_t n)
     return T2_OK;
 }
 
+// Whether the level engine sweeps with one block per angle: its tables exist
+// and every knob of the step launches is at its default (T2_NO_GRAPH asks
+// for the step launches by name).
+bool angle_form(const t2_sweeper *s)
+{
+    return s->angle_gc > 0 && s->engine == T2_ENGINE_LEVELS &&
+           s->batches == 1 && !s->concurrent && s->gpl == 1 && s->ipl == 1 &&
+           s->use_graph;
+}
+
 // psi_out = L^-1 (src + ang + ang_t).  Lagged faces read a snapshot of the
 // handle's psi taken before the sweep; a sweep into another buffer (the
 // refined solve's correction, whose previous value is zero) reads zeros
@@ -324,6 +341,24 @@ int enqueue_sweep(t2_sweeper *s, const double *ang, const void *ang_t,
         }
         return T2_OK;
     };
+    if (angle_form(s)) {
+        a.geo = geo;
+        a.topo = s->d_item_topo;
+        a.n_items = s->nc * s->na;
+        t2::AngleSweep t{};
+        t.round_off = s->d_angles;
+        t.rounds = s->d_rounds;
+        t.order = s->d_angles + s->na + 1;
+        t.items = s->d_slot_items;
+        t.lag_off = n_lag > 0 ? s->d_angles + 2 * s->na + 1 : nullptr;
+        t.n_slots = int(s->angle_slots);
+        t.zero = int(s->angle_slots + s->angle_lag);
+        t.n_angles = int(s->na);
+        t.groups = int(s->ng);
+        t.chunks = int(s->ng) / s->angle_gc;
+        T2_HIP(t2::launch_angle_sweep<T>(a, t, s->angle_block, s->stream));
+        return T2_OK;
+    }
     const int64_t nb = int64_t(s->sched.batch_steps.size()) - 1;
     if (s->engine == T2_ENGINE_LEVELS && s->concurrent && nb > 1) {
         // angle batches are independent: batch b > 0 runs on its own
@@ -596,7 +631,7 @@ int run_sweep(t2_sweeper *s, const double *ang, const void *ang_t = nullptr,
     if (s->concurrent && !s->no_alloc)   // created outside any capture
         T2_TRY(ensure_side_streams(s, n_side));
     s->n_sweeps++;
-    if (!s->use_graph)
+    if (!s->use_graph || angle_form(s))   // one launch needs no graph
         return enqueue_sweep_any(s, ang, ang_t, psi_out);
     hipGraphExec_t exec = nullptr;
     for (auto &g : s->graphs)
@@ -816,6 +851,161 @@ int build_items(t2_sweeper *s, const double *d_geo, const int4 *d_adj,
     return T2_OK;
 }
 
+void free_angle_form(t2_sweeper *s)
+{
+    dfree(s, s->d_slot_items,
+          sizeof(t2::SlotItem) * size_t(s->nc) * size_t(s->na));
+    dfree(s, s->d_rounds, sizeof(t2::AngleRound) * size_t(s->n_rounds));
+    dfree(s, s->d_angles, sizeof(int32_t) * size_t(3 * s->na + 2));
+    s->angle_gc = 0;
+}
+
+// Groups per block of the one-block-per-angle form, 0 if none will do.  The
+// table of `slots` slots has to fit the LDS, and a block's part of a vertex
+// row has to be the row or 16 bytes of it: with smaller parts the blocks of
+// an angle drift apart and psi's cache lines leave half written (93,750 cells
+// x 72 angles x 32 groups in FP64, one group a block: 18.4 ms a pass with
+// three handles at work against 8.2 ms by step launches).  Of those, the most
+// that leave kMinAngleBlocks blocks, because a block's records are read once
+// per gc groups (6,000 cells x 32 angles x 16 groups in FP64: 114, 121 and
+// 165 us a sweep with 256, 128 and 64 blocks).
+constexpr int64_t kMinAngleBlocks = 128;
+
+int angle_groups(const t2_sweeper *s, int64_t slots)
+{
+    int gc = 0;
+    for (int c = 1; c <= 8 && c <= s->ng; c *= 2)
+        if ((c == s->ng || c * s->tsize() >= 16) &&
+            t2::angle_lds_bytes(slots, c, s->tsize()) <= t2::kMaxLds &&
+            (gc == 0 || s->na * (s->ng / c) >= kMinAngleBlocks))
+            gc = c;
+    return gc;
+}
+
+// Whether that form is faster than the step launches: its bytes per solve
+// (records once per gc groups, source and psi) at the 3 TB/s it reaches
+// against 3.6 us per step and the step launches' 13.5 values per solve at
+// 5.2 TB/s.  Measured a sweep, angle form / step launches:
+//   750 cells,  32 angles, 1 group,  FP64    44 /   179 us
+//   20,250      72          1        FP32   922 /  5493 (1,703 steps)
+//   34,992     128          4        FP64   539 /  1471
+//   48,000     288          8        FP32  1897 /  2778
+//   73,002     128         16        FP32  3136 /  2819 (not taken: 2 groups)
+//   384,000    128          1        FP32  2760 /  5227
+bool angle_pays(const t2_sweeper *s, int gc)
+{
+    if (gc <= 0)
+        return false;
+    const double w = double(s->tsize());
+    const double rec = double(sizeof(t2::SlotItem)) +
+                       double(s->precision == T2_FP64
+                                  ? sizeof(t2::ItemGeo<double>)
+                                  : sizeof(t2::ItemGeo<float>));
+    const double solves = double(s->nc) * double(s->na) * double(s->ng);
+    return solves * (rec / gc + 8.0 * w) / 3.0e12 <
+           3.6e-6 * double(s->sched.n_steps) + solves * 13.5 * w / 5.2e12;
+}
+
+// Tables of the one-block-per-angle form, where it applies (before the work
+// list is released; the item records must exist).
+int build_angle_tables(t2_sweeper *s)
+{
+    const int64_t nc = s->nc, na = s->na;
+    const auto &sc = s->sched;
+    if (sc.slice.empty() || s->batches != 1 ||
+        s->gauss != T2_GAUSS_NOPIVOT ||
+        s->n_phi() * int64_t(sizeof(double)) >= (int64_t(1) << 32))
+        return T2_OK;
+    // at least about half of the widest level is live at once: do not look
+    // for slots that could not fit or would not pay
+    uint32_t width = 0;
+    for (const auto &sl : sc.slice)
+        width = std::max(width, sl.count);
+    if (!angle_pays(s, angle_groups(s, width / 2)))
+        return T2_OK;
+    std::vector<int32_t> lag_off(na + 1, 0);
+    for (const auto &l : sc.lagged)
+        lag_off[l.angle + 1]++;
+    s->angle_lag = 0;
+    for (int64_t a = 0; a < na; a++) {
+        s->angle_lag = std::max<int64_t>(s->angle_lag, lag_off[a + 1]);
+        lag_off[a + 1] += lag_off[a];
+    }
+    std::vector<uint16_t> slot;
+    T2_TRY(t2::build_slots(s->hm, na, s->omega_h.data(), sc, slot,
+                           &s->angle_slots));
+    const int64_t slots = s->angle_slots + s->angle_lag + 1;
+    const int gc = angle_groups(s, slots);
+    if (slots > t2::kMaxSlots || !angle_pays(s, gc))
+        return T2_OK;
+    const uint32_t per = 64u / uint32_t(gc);
+    std::vector<t2::AngleRound> rounds;
+    std::vector<int32_t> angles(3 * na + 2, 0);
+    int32_t *round_off = angles.data(), *order = round_off + na + 1;
+    for (int64_t a = 0; a < na; a++) {
+        uint32_t done = 0;
+        for (int32_t l = sc.lev_off[a]; l < sc.lev_off[a + 1]; l++) {
+            const t2::LevelSlice &sl = sc.slice[l];
+            const uint32_t need = done;
+            for (uint32_t i = 0; i < sl.count; i += per, done++)
+                rounds.push_back(
+                    {sl.first + i, std::min(per, sl.count - i), need});
+        }
+        round_off[a + 1] = int32_t(rounds.size());
+        order[a] = int32_t(a);
+    }
+    // deepest first, so that no long angle starts last
+    std::stable_sort(order, order + na, [&](int32_t x, int32_t y) {
+        return sc.lev_off[x + 1] - sc.lev_off[x] >
+               sc.lev_off[y + 1] - sc.lev_off[y];
+    });
+    std::copy(lag_off.begin(), lag_off.end(), order + na);
+    const size_t n_items = size_t(nc) * na;
+    s->n_rounds = int64_t(rounds.size());
+    uint16_t *d_slot = nullptr;
+    T2_TRY(dalloc_t(s, &d_slot, sizeof(uint16_t) * n_items));
+    int rc = T2_OK;
+    if ((rc = dalloc_t(s, &s->d_slot_items, sizeof(t2::SlotItem) * n_items)) ||
+        (rc = dalloc_t(s, &s->d_rounds,
+                       sizeof(t2::AngleRound) * rounds.size())) ||
+        (rc = dalloc_t(s, &s->d_angles, sizeof(int32_t) * angles.size())) ||
+        (rc = upload(s->d_rounds, rounds.data(), rounds.size())) ||
+        (rc = upload(s->d_angles, angles.data(), angles.size())) ||
+        (rc = upload(d_slot, slot.data(), slot.size()))) {
+        dfree(s, d_slot, sizeof(uint16_t) * n_items);
+        return rc;
+    }
+    hipError_t e = t2::launch_slot_items(
+        s->d_item_topo, d_slot, s->d_angles + 2 * na + 1,
+        int(s->angle_slots), int(s->angle_slots + s->angle_lag),
+        int64_t(n_items), nc, s->d_slot_items, s->stream);
+    if (e == hipSuccess)
+        e = hipStreamSynchronize(s->stream);
+    dfree(s, d_slot, sizeof(uint16_t) * n_items);
+    T2_HIP(e);
+    // enough wavefronts for a level's rounds and the preparation of the next
+    const double per_level =
+        double(rounds.size()) / double(std::max<size_t>(1, sc.slice.size()));
+    s->angle_block = per_level < 1.5 ? 256 : per_level < 3.5 ? 512 : 1024;
+    s->angle_gc = gc;
+    return T2_OK;
+}
+
+// The step launches need none of those tables: without the memory for them
+// the handle keeps to the step launches.
+int build_angle_form(t2_sweeper *s)
+{
+    const int rc = build_angle_tables(s);
+    if (rc == T2_OK && s->angle_gc > 0)
+        return T2_OK;
+    free_angle_form(s);
+    if (rc == T2_ERR_NOMEM) {
+        t2::clear_error();
+        return T2_OK;
+    }
+    return rc;
+}
+
 size_t geo_record_size(const t2_sweeper *s)
 {
     return s->precision == T2_FP64 ? sizeof(t2::ItemGeo<double>)
@@ -828,6 +1018,7 @@ void free_schedule(t2_sweeper *s)
     const int64_t n_lag = int64_t(s->sched.lagged.size());
     drop_graphs(s);
     free_queue(s);
+    free_angle_form(s);
     dfree(s, s->d_item_geo, geo_record_size(s) * n_items);
     dfree(s, s->d_item_geo64, sizeof(t2::ItemGeo<double>) * n_items);
     dfree(s, s->d_item_topo, sizeof(t2::ItemTopo) * n_items);
@@ -902,7 +1093,6 @@ int build_schedule_device(t2_sweeper *s)
         cleanup();
         return rc;
     }
-    std::vector<uint32_t>().swap(s->sched.work);
     if (s->precision == T2_FP64) {
         rc = build_items<double>(
             s, d_geo, d_adj, d_work, d_sig_cell,
@@ -920,6 +1110,9 @@ int build_schedule_device(t2_sweeper *s)
                                      s->d_item_geo64);
     }
     cleanup();
+    if (rc == T2_OK)
+        rc = build_angle_form(s);
+    std::vector<uint32_t>().swap(s->sched.work);
     return rc;
 }
 

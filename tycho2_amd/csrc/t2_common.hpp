@@ -50,6 +50,12 @@ struct LaggedFace {
     int32_t upwind;
 };
 
+// A run of consecutive items of the step-ordered work list.
+struct LevelSlice {
+    uint32_t first;
+    uint32_t count;
+};
+
 // Sweep schedule: every (angle, cell) pair in level order.
 struct Schedule {
     int64_t n_steps = 0;
@@ -59,6 +65,11 @@ struct Schedule {
     std::vector<uint32_t> work;        // [nc * na]
     std::vector<LaggedFace> lagged;    // sorted by (angle, cell, face)
     std::vector<int64_t> batch_steps;  // angle batch b: steps [b], [b + 1]
+    // Level sets only (empty for a priority schedule): the items of angle a
+    // at its level l are slice[lev_off[a] + l], a contiguous range of the
+    // work list.
+    std::vector<int32_t> lev_off;      // [na + 1]
+    std::vector<LevelSlice> slice;     // [lev_off[na]]
 };
 
 // Dependency rule of the level sets.  dep_tol < 0: the graph traverser's,
@@ -90,6 +101,14 @@ std::vector<int32_t> angle_batches(int64_t na, const double *omega,
 int build_schedule(const HostMesh &m, int64_t na, const double *omega,
                    int batches, int order, Schedule &s,
                    double dep_tol = kTraverseRule);
+
+// Slot of every (angle, cell) in its angle's table of live psi values
+// (level-set schedules, before the work list is released); *n_slots is the
+// largest table of any angle (slots are valid when it is below kNoSlot).
+constexpr uint16_t kNoSlot = 0xFFFF;
+int build_slots(const HostMesh &m, int64_t na, const double *omega,
+                const Schedule &s, std::vector<uint16_t> &slot,
+                int64_t *n_slots);
 
 // Traversal priorities of the reference's graph traverser on one rank
 // (src/Priorities.cc:396-435): intra-angle rule 0 random, 1 b-level,

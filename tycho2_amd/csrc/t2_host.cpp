@@ -363,9 +363,16 @@ int build_schedule(const HostMesh &m, int64_t na, const double *omega,
         s.step_off[st + 1] += s.step_off[st];
     std::vector<int64_t> pos(s.step_off.begin(), s.step_off.end() - 1);
     s.work.resize(size_t(na) * nc);
+    s.lev_off.assign(na + 1, 0);
+    for (int64_t a = 0; a < na; a++)
+        s.lev_off[a + 1] = s.lev_off[a] + nlev[a];
+    s.slice.resize(s.lev_off[na]);
     std::vector<int32_t> cells(nc);
     for (int64_t a = 0; a < na; a++) {
         const int32_t *l = levels.data() + a * nc;
+        LevelSlice *sl = s.slice.data() + s.lev_off[a];
+        for (int32_t lev = 0; lev < nlev[a]; lev++)
+            sl[lev].first = uint32_t(pos[boff[batch[a]] + lev]);
         for (int64_t c = 0; c < nc; c++)
             cells[c] = int32_t(c);
         if (order == T2_ORDER_FACES) {
@@ -393,6 +400,9 @@ int build_schedule(const HostMesh &m, int64_t na, const double *omega,
             s.work[pos[boff[batch[a]] + l[c]]++] =
                 uint32_t(c) | (uint32_t(a) << cb);
         }
+        for (int32_t lev = 0; lev < nlev[a]; lev++)
+            sl[lev].count = uint32_t(pos[boff[batch[a]] + lev]) -
+                            sl[lev].first;
     }
     return T2_OK;
 }
@@ -417,6 +427,78 @@ void for_each_angle(int64_t na, F body)
     for (auto &t : pool)
         t.join();
 }
+
+}  // namespace
+
+// Live psi values of each angle's sweep as slots of a small table: a cell
+// holds its slot from its own level to its last reader's, and a slot is
+// handed on to a cell of a later level (a level's readers and writers run
+// together).  slot[a * nc + c], kNoSlot where no cell reads (a, c).
+int build_slots(const HostMesh &m, int64_t na, const double *omega,
+                const Schedule &s, std::vector<uint16_t> &slot,
+                int64_t *n_slots)
+{
+    const int64_t nc = m.nc;
+    const uint32_t cmask = (uint32_t(1) << s.cell_bits) - 1;
+    try {
+        slot.assign(size_t(na) * nc, kNoSlot);
+    } catch (...) {
+        return fail(T2_ERR_NOMEM, "host memory for the sweep's slots");
+    }
+    std::vector<int64_t> most(na, 0);
+    for_each_angle(na, [&](int64_t a) {
+        const double *om = omega + 3 * a;
+        const LevelSlice *sl = s.slice.data() + s.lev_off[a];
+        const int32_t nlev = s.lev_off[a + 1] - s.lev_off[a];
+        uint16_t *mine = slot.data() + a * nc;
+        // last level reading each cell (-1: none)
+        std::vector<int32_t> last(nc, -1);
+        std::vector<uint8_t> lagged(nc, 0);
+        auto lo = std::lower_bound(
+            s.lagged.begin(), s.lagged.end(), a,
+            [](const LaggedFace &f, int64_t x) { return f.angle < x; });
+        for (; lo != s.lagged.end() && lo->angle == a; ++lo)
+            lagged[lo->cell] |= uint8_t(1u << lo->face);
+        for (int32_t l = 0; l < nlev; l++)
+            for (uint32_t i = 0; i < sl[l].count; i++) {
+                const int64_t c = s.work[sl[l].first + i] & cmask;
+                for (int k = 0; k < 4; k++) {
+                    const int64_t u = m.adj[4 * c + k];
+                    if (u >= 0 && !(lagged[c] >> k & 1u) &&
+                        omega_dot_n(om, &m.normal[(4 * c + k) * 3]) < 0)
+                        last[u] = std::max(last[u], l);
+                }
+            }
+        // cells whose slot is free again after level l, as linked lists
+        std::vector<int32_t> head(nlev, -1), next(nc, -1);
+        std::vector<uint16_t> spare;
+        int64_t used = 0;
+        for (int32_t l = 0; l < nlev; l++) {
+            if (l > 0)
+                for (int32_t c = head[l - 1]; c >= 0; c = next[c])
+                    spare.push_back(mine[c]);
+            for (uint32_t i = 0; i < sl[l].count; i++) {
+                const int32_t c = int32_t(s.work[sl[l].first + i] & cmask);
+                if (last[c] < 0)
+                    continue;
+                if (!spare.empty()) {
+                    mine[c] = spare.back();
+                    spare.pop_back();
+                } else {
+                    mine[c] = uint16_t(std::min<int64_t>(used, kNoSlot));
+                    used++;
+                }
+                next[c] = head[last[c]];
+                head[last[c]] = c;
+            }
+        }
+        most[a] = used;
+    });
+    *n_slots = *std::max_element(most.begin(), most.end());
+    return T2_OK;
+}
+
+namespace {
 
 // The sweep dependency graph of every direction as the level sets resolve
 // it: (a, c) -> (a, u) when face k of c is outgoing (Omega.n > 0, the
@@ -717,6 +799,8 @@ int build_priority_schedule(const HostMesh &m, int64_t na,
                                 "items unscheduled");
     s.n_steps = int64_t(s.step_off.size()) - 1;
     s.batch_steps = {0, s.n_steps};
+    s.lev_off.clear();
+    s.slice.clear();
     return T2_OK;
 }
 

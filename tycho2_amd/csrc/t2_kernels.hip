@@ -10,6 +10,8 @@
 #include "t2_kernels.hpp"
 
 #include <algorithm>
+#include <cmath>
+#include <type_traits>
 
 namespace t2 {
 namespace {
@@ -494,46 +496,125 @@ __device__ __forceinline__ void load_item(const SweepArgs<T> &p, int64_t item,
     }
 }
 
-// The cell solve of solve_item on preloaded inputs (same arithmetic, same
-// order), and the store of psi.
+// The cell solve of solve_item in two parts, so that everything that does
+// not read upwind psi can be done ahead: the factors of the cell's matrix
+// with the source's right-hand side, then the upwind faces and the two
+// triangular solves.  Same arithmetic and order as solve_item; every fused
+// multiply-add is written out, because the compiler fuses across statements
+// only within a basic block and the two forms differ in their branches.
+template <typename T>
+struct CellFactors {
+    T low[4][3];       // column r below the pivot, before row r is scaled
+    T up[3][4];        // row r right of the pivot, scaled
+    T inv[4];          // reciprocal pivots
+    T b[4];            // right-hand side
+};
+
+template <typename T>
+__device__ __forceinline__ void factor_cell(const T a12[4], T v20, T sig,
+                                            const T q[4], CellFactors<T> &f)
+{
+#pragma clang fp contract(off)
+    T o[4];
+    T P = T(0);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        o[k] = a12[k] > T(0) ? a12[k] : T(0);
+        P += o[k];
+    }
+    const T sumq = (q[0] + q[1]) + (q[2] + q[3]);
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+        f.b[v] = v20 * (sumq + q[v]);
+    T m[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const T rest = P - o[i];
+        const T base = __builtin_elementwise_fma(sig, v20, a12[i]);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            m[i][j] = (i == j)
+                          ? __builtin_elementwise_fma(
+                                T(2),
+                                __builtin_elementwise_fma(sig, v20, rest),
+                                a12[i])
+                          : base + (rest - o[j]);
+    }
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        f.inv[r] = recip<T>(m[r][r]);
+#pragma unroll
+        for (int c = r + 1; c < 4; c++)
+            f.up[r][c] = m[r][c] * f.inv[r];
+#pragma unroll
+        for (int row = r + 1; row < 4; row++) {
+            f.low[row][r] = m[row][r];
+#pragma unroll
+            for (int c = r + 1; c < 4; c++)
+                m[row][c] = __builtin_elementwise_fma(-f.up[r][c], m[row][r],
+                                                      m[row][c]);
+        }
+    }
+    f.inv[3] = recip<T>(m[3][3]);
+}
+
+// Upwind face k: b_i -= a_k (sum_j u_j + u_i), i != k (u_k = 0).
+template <typename T>
+__device__ __forceinline__ void add_face(T a, int k, const T uv[4], T b[4])
+{
+#pragma clang fp contract(off)
+    const T sum = (uv[0] + uv[1]) + (uv[2] + uv[3]);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (i != k)
+            b[i] = __builtin_elementwise_fma(-a, sum + uv[i], b[i]);
+}
+
+template <typename T>
+__device__ __forceinline__ void substitute(const CellFactors<T> &f, T b[4])
+{
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        b[r] *= f.inv[r];
+#pragma unroll
+        for (int row = r + 1; row < 4; row++)
+            b[row] = __builtin_elementwise_fma(-b[r], f.low[row][r], b[row]);
+    }
+    b[3] *= f.inv[3];
+#pragma unroll
+    for (int r = 2; r >= 0; r--)
+#pragma unroll
+        for (int c = 3; c > r; c--)
+            b[r] = __builtin_elementwise_fma(-f.up[r][c], b[c], b[r]);
+}
+
+// The cell solve of solve_item on preloaded inputs: b = psi at the cell's
+// vertices.
+template <typename T>
+__device__ __forceinline__ void solve_loaded(const ItemLoad<T> &in, T b[4])
+{
+    CellFactors<T> f;
+    factor_cell<T>(in.a12, in.v20, in.sig, in.q, f);
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+        b[v] = f.b[v];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        if (in.up[k] != -1)
+            add_face<T>(in.a12[k], k, in.uw[k], b);
+    substitute<T>(f, b);
+}
+
+// ... and the store of psi.
 template <typename T, int G>
 __device__ __forceinline__ void solve_store_item(const SweepArgs<T> &p,
                                                  int64_t item, int g,
                                                  const ItemLoad<T> &in)
 {
     constexpr uint32_t CG = 4 * G;
-    T o[4];
-    T P = T(0);
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        o[k] = in.a12[k] > T(0) ? in.a12[k] : T(0);
-        P += o[k];
-    }
-    const T s = in.sig * in.v20;
-    const T sumq = (in.q[0] + in.q[1]) + (in.q[2] + in.q[3]);
     T b[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++)
-        b[v] = in.v20 * (sumq + in.q[v]);
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        if (in.up[k] == -1)
-            continue;
-        const T *uv = in.uw[k];
-        const T sum = (uv[0] + uv[1]) + (uv[2] + uv[3]);
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            if (i != k)
-                b[i] -= in.a12[k] * (sum + uv[i]);
-    }
-    T m[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            m[i][j] = (i == j) ? in.a12[i] + T(2) * (s + (P - o[i]))
-                               : in.a12[i] + s + ((P - o[i]) - o[j]);
-    solve_nopivot<T>(m, b);
+    solve_loaded<T>(in, b);
     const ItemTopo t = p.topo[item];
     T *dst = p.psi + size_t(t.angle) * size_t(p.nc) * CG +
              uint32_t(t.cell) * CG + g;
@@ -572,6 +653,388 @@ sweep_step2_kernel(const SweepArgs<T> p)
     solve_store_item<T, G>(p, a, g, in_a);
     if (has_b)
         solve_store_item<T, G>(p, b, g, in_b);
+}
+
+// ------------------------------------------------------ one block per angle
+using Word2 = uint32_t __attribute__((ext_vector_type(2)));
+using Word4 = uint32_t __attribute__((ext_vector_type(4)));
+using Rsrc = __amdgpu_buffer_rsrc_t;
+
+// Buffer descriptor of `bytes` bytes at p (both uniform): loads past the end
+// return zero and stores past it are dropped, so lanes without an item need
+// no branch around their memory accesses.
+__device__ __forceinline__ Rsrc buffer_of(const void *p, uint32_t bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes,
+                                             0x00027000);
+}
+
+constexpr uint32_t kOutside = 0xFFFFFFFFu;   // offset past every buffer's end
+constexpr uint32_t kMaxPolls = 1u << 26;
+
+__device__ __forceinline__ void buffer_value(Rsrc r, uint32_t off, double &x)
+{
+    x = __builtin_bit_cast(double,
+                           __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+}
+__device__ __forceinline__ void buffer_value(Rsrc r, uint32_t off, float &x)
+{
+    x = __builtin_bit_cast(float,
+                           __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+}
+__device__ __forceinline__ void buffer_store(Rsrc r, uint32_t off, double x)
+{
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(Word2, x), r, off,
+                                          0, 0);
+}
+__device__ __forceinline__ void buffer_store(Rsrc r, uint32_t off, float x)
+{
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), r,
+                                          off, 0, 0);
+}
+// Four contiguous values.  An offset of kOutside stays outside when the
+// second half's 16 bytes are added to it: the hardware compares without
+// wrapping, but the sum here is 32-bit, so it is not formed from kOutside.
+__device__ __forceinline__ void buffer_row(Rsrc r, uint32_t off, double x[4])
+{
+    struct W {
+        Word4 w[2];
+    } t;
+    t.w[0] = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+    t.w[1] = __builtin_amdgcn_raw_buffer_load_b128(
+        r, off == kOutside ? off : off + 16, 0, 0);
+    struct X {
+        double v[4];
+    } y = __builtin_bit_cast(X, t);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        x[i] = y.v[i];
+}
+__device__ __forceinline__ void buffer_row(Rsrc r, uint32_t off, float x[4])
+{
+    struct X {
+        float v[4];
+    } y = __builtin_bit_cast(
+        X, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        x[i] = y.v[i];
+}
+__device__ __forceinline__ void buffer_store_row(Rsrc r, uint32_t off,
+                                                 const double x[4])
+{
+    struct X {
+        double v[4];
+    } y = {{x[0], x[1], x[2], x[3]}};
+    struct W {
+        Word4 w[2];
+    } t = __builtin_bit_cast(W, y);
+    __builtin_amdgcn_raw_buffer_store_b128(t.w[0], r, off, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(
+        t.w[1], r, off == kOutside ? off : off + 16, 0, 0);
+}
+__device__ __forceinline__ void buffer_store_row(Rsrc r, uint32_t off,
+                                                 const float x[4])
+{
+    struct X {
+        float v[4];
+    } y = {{x[0], x[1], x[2], x[3]}};
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(Word4, y), r,
+                                           off, 0, 0);
+}
+__device__ __forceinline__ void buffer_geo(Rsrc r, uint32_t off,
+                                           ItemGeo<double> &g)
+{
+    struct W {
+        Word4 w[3];
+    } x;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+        x.w[i] = __builtin_amdgcn_raw_buffer_load_b128(r, off + 16 * i, 0, 0);
+    g = __builtin_bit_cast(ItemGeo<double>, x);
+}
+__device__ __forceinline__ void buffer_geo(Rsrc r, uint32_t off,
+                                           ItemGeo<float> &g)
+{
+    struct W {
+        Word4 a;
+        Word2 b;
+    } x;
+    x.a = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+    x.b = __builtin_amdgcn_raw_buffer_load_b64(r, off + 16, 0, 0);
+    g = __builtin_bit_cast(ItemGeo<float>, x);
+}
+
+// A block sweeps one angle for GC groups; the values that later levels read
+// stay in the block's LDS (slot form of the records), so that a level hands
+// on to the next without a global round trip.
+//
+// The angle's items are cut into rounds of one wavefront (64 / GC items, a
+// round never spans two levels), dealt out to the wavefronts in turn.  A
+// wavefront loads its next round's inputs and factors its cells' matrices
+// while earlier rounds run, then waits until every round of the earlier
+// levels is done (a counter in LDS), adds the upwind faces, substitutes and
+// stores.  So only the upwind reads and the substitution are on the path from
+// level to level.  Rounds are taken in ascending order by resident
+// wavefronts: the lowest unfinished one never waits.  (A wait that ran past
+// kMaxPolls all the same would leave NaN in psi.)
+//
+// The wavefront's LDS operations are performed in order, so a round's values
+// are in LDS before its count is.
+//
+// ANG: angle-dependent source, 0 none, 1 FP64 (src_ang), 2 T (src_ang_t).
+// ROW: one group in all, so that a cell's four values are contiguous and move
+// in one access.
+template <typename T, int GC, int ANG, bool ROW>
+__global__ void __launch_bounds__(kMaxAngleBlock)
+angle_sweep_kernel(const SweepArgs<T> p, const AngleSweep t)
+{
+    extern __shared__ char lds_raw[];
+    int32_t *const done = reinterpret_cast<int32_t *>(lds_raw);
+    T *const live = reinterpret_cast<T *>(lds_raw + kAngleLdsHead);
+    const int x = int(blockIdx.x % kXcds), j = int(blockIdx.x / kXcds);
+    const int ai = (j / t.chunks) * kXcds + x;
+    if (ai >= t.n_angles)
+        return;
+    const int angle = t.order[ai];
+    const uint32_t lane = threadIdx.x % 64;
+    const uint32_t lg = lane % GC, li = lane / GC;
+    const uint32_t G = uint32_t(t.groups), CG = 4 * G;
+    const uint32_t g = uint32_t(j % t.chunks) * GC + lg;
+    const size_t plane = size_t(p.nc) * CG;
+    const uint32_t plane_bytes = uint32_t(plane * sizeof(T));
+    const Rsrc psi_a = buffer_of(p.psi + size_t(angle) * plane, plane_bytes);
+    const Rsrc src = buffer_of(p.src_iso, plane_bytes);
+    const Rsrc src_a =
+        ANG == 1 ? buffer_of(p.src_ang + size_t(angle) * plane,
+                             uint32_t(plane * sizeof(double)))
+                 : buffer_of(ANG == 2 ? p.src_ang_t + size_t(angle) * plane
+                                      : nullptr,
+                             ANG == 2 ? plane_bytes : 0u);
+    const bool by_item = p.sigma_mode == kSigmaCellGroup;
+    const Rsrc sigma =
+        buffer_of(p.sigma, by_item ? uint32_t(p.nc * G * sizeof(T)) : 0u);
+    const T sig_g = p.sigma_mode == kSigmaGroup ? p.sigma[g] : T(0);
+
+    // after the live slots: the pre-sweep values of the angle's lagged faces
+    // and a slot of zeros, which the faces that read nothing name
+    if (threadIdx.x == 0)
+        *done = 0;
+    if (threadIdx.x < 4 * GC)
+        live[size_t(t.zero) * 4 * GC + threadIdx.x] = T(0);
+    if (t.lag_off) {
+        const int lag0 = t.lag_off[angle];
+        const int n = (t.lag_off[angle + 1] - lag0) * 4 * GC;
+        for (int i = int(threadIdx.x); i < n; i += int(blockDim.x))
+            live[size_t(t.n_slots) * 4 * GC + i] =
+                p.lag_buf[(size_t(lag0) * 4 + i / GC) * G + g];
+    }
+    __syncthreads();
+
+    const int n_rounds = t.round_off[angle + 1] - t.round_off[angle];
+    const AngleRound *const rounds = t.rounds + t.round_off[angle];
+    const int n_waves = int(blockDim.x / 64);
+    int k = __builtin_amdgcn_readfirstlane(int(threadIdx.x / 64));
+    struct Record {
+        Word4 a, b;                // a SlotItem
+    };
+    struct Inputs {
+        ItemGeo<T> geo;
+        T sig, q[4];
+        std::conditional_t<ANG == 1, double, T> qa[4];
+    };
+    auto round_at = [&](int i) {
+        AngleRound r{0, 0, 0};
+        if (i < n_rounds)
+            r = rounds[i];
+        return r;
+    };
+    auto load_record = [&](const AngleRound &r) {
+        const Rsrc b = buffer_of(t.items + r.item,
+                                 r.count * uint32_t(sizeof(SlotItem)));
+        Record rec;
+        rec.a = __builtin_amdgcn_raw_buffer_load_b128(
+            b, li * uint32_t(sizeof(SlotItem)), 0, 0);
+        rec.b = __builtin_amdgcn_raw_buffer_load_b128(
+            b, li * uint32_t(sizeof(SlotItem)) + 16u, 0, 0);
+        return rec;
+    };
+    auto load_inputs = [&](const AngleRound &r, const Record &rec,
+                           Inputs &in) {
+        const Rsrc b = buffer_of(p.geo + r.item,
+                                 r.count * uint32_t(sizeof(ItemGeo<T>)));
+        buffer_geo(b, li * uint32_t(sizeof(ItemGeo<T>)), in.geo);
+        const bool mine = li < r.count;
+        const uint32_t cell = rec.a[0];
+        if (by_item)
+            buffer_value(sigma,
+                         mine ? (cell * G + g) * uint32_t(sizeof(T))
+                              : kOutside,
+                         in.sig);
+        if constexpr (ROW) {
+            buffer_row(src, mine ? cell * 4 * uint32_t(sizeof(T)) : kOutside,
+                       in.q);
+            if constexpr (ANG != 0)
+                buffer_row(src_a,
+                           mine ? cell * 4 * uint32_t(sizeof(in.qa[0]))
+                                : kOutside,
+                           in.qa);
+            return;
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const uint32_t e = cell * CG + g + v * G;
+            buffer_value(src, mine ? e * uint32_t(sizeof(T)) : kOutside,
+                         in.q[v]);
+            if constexpr (ANG != 0)
+                buffer_value(src_a,
+                             mine ? e * uint32_t(sizeof(in.qa[0])) : kOutside,
+                             in.qa[v]);
+        }
+    };
+
+    // FP32 issues the next inputs before it waits and reads every face's
+    // values at once; in FP64 the inputs would not fit beside the factors
+    // (128 registers for 16 wavefronts a block), and skipping the faces that
+    // no lane reads pays for its branch
+    constexpr bool kEarly = sizeof(T) == 4;
+    AngleRound r0 = round_at(k), r1 = round_at(k + n_waves);
+    Record rec0 = load_record(r0), rec1 = load_record(r1);
+    Inputs in;
+    load_inputs(r0, rec0, in);
+    for (; k < n_rounds; k += n_waves) {
+        // ahead of the earlier levels: this round's factors and LDS
+        // addresses, the next one's inputs, the record of the one after it
+        T a12[4], q[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            a12[i] = in.geo.a12[i];
+            q[i] = in.q[i];
+            if constexpr (ANG != 0)
+                q[i] += T(in.qa[i]);
+        }
+        CellFactors<T> f;
+        factor_cell<T>(a12, in.geo.v20,
+                       by_item ? in.sig
+                       : p.sigma_mode == kSigmaGroup ? sig_g
+                                                     : in.geo.sig,
+                       q, f);
+        uint32_t at[12];
+#pragma unroll
+        for (int i = 0; i < 12; i++) {
+            const uint32_t w = i < 4 ? rec0.a[2 + i / 2] : rec0.b[i / 2 - 2];
+            at[i] = (i % 2 ? w >> 16 : w & 0xFFFFu) * GC + lg;
+        }
+        const bool mine = li < r0.count;
+        const uint32_t own = mine ? rec0.a[1] & 0xFFFFu : uint32_t(kNoValue);
+        const uint32_t dst = (rec0.a[0] * CG + g) * uint32_t(sizeof(T));
+        const int need = int(r0.need);
+        // faces that any lane of the wavefront reads
+        bool reads[4];
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++)
+            reads[kk] = kEarly || __any(mine && at[3 * kk] <
+                                                    uint32_t(t.zero) * 4 * GC);
+        r0 = r1;
+        r1 = round_at(k + 2 * n_waves);
+        rec0 = rec1;
+        if constexpr (kEarly)
+            load_inputs(r0, rec0, in);
+        rec1 = load_record(r1);
+
+        uint32_t polls = 0;
+        while (__builtin_amdgcn_readfirstlane(__hip_atomic_load(
+                   done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) <
+               need) {
+            if (++polls == kMaxPolls) {   // cannot happen; seconds
+                f.inv[3] = T(NAN);
+                break;
+            }
+        }
+        asm volatile("" ::: "memory");   // no LDS read above the wait
+        // the wavefront whose turn it is goes before those preparing
+        __builtin_amdgcn_s_setprio(3);
+        T uv[12];
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++)
+            if (reads[kk]) {
+                uv[3 * kk] = live[at[3 * kk]];
+                uv[3 * kk + 1] = live[at[3 * kk + 1]];
+                uv[3 * kk + 2] = live[at[3 * kk + 2]];
+            }
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) {
+            if (!reads[kk])
+                continue;
+            T u[4];
+            int slot = 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                u[i] = i == kk ? T(0) : uv[3 * kk + slot++];
+            add_face<T>(a12[kk], kk, u, f.b);
+        }
+        substitute<T>(f, f.b);
+        if (own != kNoValue) {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                live[(own + v) * GC + lg] = f.b[v];
+        }
+        asm volatile("" ::: "memory");   // no LDS write below the count
+        if (lane == 0)
+            __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+        __builtin_amdgcn_s_setprio(0);
+        // plain stores: the other chunks' blocks complete the cache lines
+        if constexpr (ROW) {
+            buffer_store_row(psi_a, mine ? dst : kOutside, f.b);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                buffer_store(psi_a,
+                             mine ? dst + v * G * uint32_t(sizeof(T))
+                                  : kOutside,
+                             f.b[v]);
+        }
+        if constexpr (!kEarly)
+            load_inputs(r0, rec0, in);
+    }
+}
+
+// Records of the slot form of every item.
+__global__ void slot_items_kernel(const ItemTopo *__restrict__ topo,
+                                  const uint16_t *__restrict__ slot,
+                                  const int32_t *__restrict__ lag_off,
+                                  int n_slots, int zero, int64_t n, int64_t nc,
+                                  SlotItem *__restrict__ out)
+{
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= n)
+        return;
+    const ItemTopo t = topo[i];
+    const uint16_t *mine = slot + size_t(t.angle) * size_t(nc);
+    SlotItem o;
+    o.cell = uint32_t(t.cell);
+    const uint32_t own = mine[t.cell];
+    o.own = own == 0xFFFFu ? kNoValue : uint16_t(own * 4);
+    o.pad = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int32_t u = t.up[k];
+        int s = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (j == k)
+                continue;
+            uint32_t at = uint32_t(zero) * 4;     // contributes nothing
+            if (u >= 0)
+                at = uint32_t(mine[u]) * 4 + ((t.meta >> (6 * k + 2 * s)) & 3u);
+            else if (u < -1)   // lagged: the item's own vertex order
+                at = uint32_t(n_slots + (-2 - u) - lag_off[t.angle]) * 4 + j;
+            o.in[3 * k + s] = uint16_t(at);
+            s++;
+        }
+    }
+    out[i] = o;
 }
 
 // ---------------------------------------------------------------- ready queue
@@ -1271,6 +1734,73 @@ hipError_t launch_sweep_step(const SweepArgs<T> &args, int groups,
     }
 }
 
+template <typename T, int GC, int ANG, bool ROW>
+hipError_t launch_angle_k(const SweepArgs<T> &args, const AngleSweep &t,
+                          int block, size_t lds, hipStream_t stream)
+{
+    const hipError_t e = hipFuncSetAttribute(
+        reinterpret_cast<const void *>(&angle_sweep_kernel<T, GC, ANG, ROW>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, int(kMaxLds));
+    if (e != hipSuccess)
+        return e;
+    const unsigned grid =
+        unsigned((t.n_angles + kXcds - 1) / kXcds * kXcds * t.chunks);
+    hipLaunchKernelGGL((angle_sweep_kernel<T, GC, ANG, ROW>), dim3(grid),
+                       dim3(block), lds, stream, args, t);
+    return hipGetLastError();
+}
+
+template <typename T, int GC, bool ROW>
+hipError_t launch_angle_g(const SweepArgs<T> &args, const AngleSweep &t,
+                          int block, size_t lds, hipStream_t stream)
+{
+    if (args.src_ang)
+        return launch_angle_k<T, GC, 1, ROW>(args, t, block, lds, stream);
+    if constexpr (sizeof(T) == 4)
+        if (args.src_ang_t)
+            return launch_angle_k<T, GC, 2, ROW>(args, t, block, lds, stream);
+    return launch_angle_k<T, GC, 0, ROW>(args, t, block, lds, stream);
+}
+
+template <typename T>
+hipError_t launch_angle_sweep(const SweepArgs<T> &args, const AngleSweep &t,
+                              int block, hipStream_t stream)
+{
+    const int gc = t.chunks > 0 ? t.groups / t.chunks : 0;
+    const size_t lds = angle_lds_bytes(t.zero + 1, gc, sizeof(T));
+    // the kernel's byte offsets within a plane are 32-bit, below kOutside
+    const int64_t plane = args.nc * 4 * t.groups * int64_t(sizeof(double));
+    if (block < 64 || block > kMaxAngleBlock || block % 64 || lds > kMaxLds ||
+        gc * t.chunks != t.groups || t.n_angles <= 0 || t.zero >= kMaxSlots ||
+        plane >= (int64_t(1) << 32) || args.solver != kSolveNoPivot ||
+        args.problems || args.active || (args.src_ang && args.src_ang_t) ||
+        (sizeof(T) == 8 && args.src_ang_t))
+        return hipErrorInvalidValue;
+    switch (gc) {
+    case 1:
+        return t.groups == 1
+                   ? launch_angle_g<T, 1, true>(args, t, block, lds, stream)
+                   : launch_angle_g<T, 1, false>(args, t, block, lds, stream);
+    case 2: return launch_angle_g<T, 2, false>(args, t, block, lds, stream);
+    case 4: return launch_angle_g<T, 4, false>(args, t, block, lds, stream);
+    case 8: return launch_angle_g<T, 8, false>(args, t, block, lds, stream);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t launch_slot_items(const ItemTopo *topo, const uint16_t *slot,
+                             const int32_t *lag_off, int n_slots, int zero,
+                             int64_t n, int64_t nc, SlotItem *out,
+                             hipStream_t stream)
+{
+    if (n <= 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(slot_items_kernel, dim3(unsigned((n + 255) / 256)),
+                       dim3(256), 0, stream, topo, slot, lag_off, n_slots,
+                       zero, n, nc, out);
+    return hipGetLastError();
+}
+
 template <typename T, int G, int GPL>
 hipError_t queue_dispatch(const SweepArgs<T> *args, const QueueState *q,
                           int block, int64_t grid, hipStream_t stream,
@@ -1581,6 +2111,9 @@ hipError_t launch_fill(double *x, double v, int64_t n, hipStream_t stream)
         hipStream_t);                                                         \
     template hipError_t launch_sweep_step<T>(const SweepArgs<T> &, int, int,  \
                                              int, hipStream_t);               \
+    template hipError_t launch_angle_sweep<T>(const SweepArgs<T> &,           \
+                                              const AngleSweep &, int,        \
+                                              hipStream_t);                   \
     template hipError_t launch_residual<T>(const ResidualArgs<T> &, int,      \
                                            hipStream_t);                      \
     template hipError_t launch_queue_sweep<T>(const SweepArgs<T> &,           \

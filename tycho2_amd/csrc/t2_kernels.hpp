@@ -140,6 +140,53 @@ hipError_t launch_sweep_step(const SweepArgs<T> &args, int groups,
                              int groups_per_lane, int block,
                              hipStream_t stream);
 
+// One block per (angle, chunk of groups): the angle's items in rounds of one
+// wavefront, level by level.
+constexpr int kMaxAngleBlock = 1024;
+constexpr size_t kMaxLds = 160 * 1024;
+constexpr size_t kAngleLdsHead = 16;   // the block's count of finished rounds
+struct AngleRound {
+    uint32_t item, count;          // work items
+    uint32_t need;                 // rounds of the angle's earlier levels
+};
+// Slot form of an item's record: its values' place in the angle's table of
+// live values (4 per slot; kNoValue: no cell reads them), and for each face
+// the places of the three upwind values facing the cell's vertices other
+// than the face's own (a slot of zeros where the face reads nothing).
+constexpr uint16_t kNoValue = 0xFFFF;
+constexpr int kMaxSlots = 0x3FFE;      // slots x 4 + vertex in 16 bits
+struct alignas(16) SlotItem {
+    uint32_t cell;
+    uint16_t own, pad;
+    uint16_t in[12];
+};
+struct AngleSweep {
+    const int32_t *round_off;      // [n_angles + 1] rounds of an angle
+    const AngleRound *rounds;
+    const int32_t *order;          // [n_angles] angles, most rounds first
+    const SlotItem *items;         // slot form of the records
+    const int32_t *lag_off;        // [n_angles + 1] lagged faces, or null
+    int n_slots;                   // slots of the live values' table
+    int zero;                      // its slot of zeros (after the lagged ones)
+    int n_angles;
+    int groups;
+    int chunks;                    // blocks per angle (groups split evenly)
+};
+
+// LDS of a block: its count and a table of `slots` slots for gc groups.
+inline size_t angle_lds_bytes(int64_t slots, int gc, size_t value)
+{
+    return kAngleLdsHead + size_t(slots) * 4 * size_t(gc) * value;
+}
+
+template <typename T>
+hipError_t launch_angle_sweep(const SweepArgs<T> &args, const AngleSweep &t,
+                              int block, hipStream_t stream);
+hipError_t launch_slot_items(const ItemTopo *topo, const uint16_t *slot,
+                             const int32_t *lag_off, int n_slots, int zero,
+                             int64_t n, int64_t nc, SlotItem *out,
+                             hipStream_t stream);
+
 // Ready-queue form of a sweep: one persistent launch over the step-ordered
 // items from first_item on, split into chunks that never span two steps.
 // The queued items' tables are indexed by item - first_item.
