@@ -396,7 +396,9 @@ int t2_sweep_only(t2_sweeper *s);
  *   T2_ENGINE_LEVELS  members with the same group count share one merged
  *                     step schedule (one launch per merged step and group
  *                     count, replayed from a hipGraph); the merged records
- *                     are a copy of the members' records;
+ *                     are a copy of the members' records; members small or
+ *                     deep enough for it are swept with one block per angle,
+ *                     all of them in one or two launches;
  *   T2_ENGINE_QUEUE   one persistent launch for all members: chunks of the
  *                     members' items interleaved step by step behind one
  *                     ticket counter, each waiting on its own problem's

@@ -6,7 +6,7 @@ import pytest
 
 from tycho2_amd import mesh as meshmod
 from tycho2_amd.quadrature import product_quadrature
-from tycho2_amd.sweeper import FP32, FP64, SweeperHIP
+from tycho2_amd.sweeper import FP32, FP64, SweepBatch, SweeperHIP
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +64,50 @@ def test_equals_step_launches(n, sn, ng, sigma, precision, monkeypatch):
     for a, b in zip(got, ref):
         assert np.isfinite(a).all()
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("chains", [0, 1, 2])
+@pytest.mark.parametrize("precision", [FP64, FP32])
+def test_batch_of_both_forms(precision, chains):
+    """Members swept with one block per angle beside members that only the
+    merged step launches take (a priority schedule): each as by itself."""
+    print(f"angle form batch precision={precision} chains={chains}",
+          flush=True)
+    shapes = [(3, 4, 1, False), (4, 4, 8, True), (5, 8, 2, False),
+              (4, 2, 16, False), (3, 4, 8, True), (6, 4, 4, False)]
+
+    def members():
+        out = []
+        for i, (n, sn, ng, steps) in enumerate(shapes):
+            s = handle(n, sn, ng, precision, "both", seed=20 + i)
+            if steps:
+                s.set_priority(1, 0, 0)
+            out.append(s)
+        return out
+
+    ref = []
+    for s in members():
+        with s:
+            s.solve_krylov(200, 1e-9 if precision == FP64 else 1e-5, 20)
+            s.sweep_step()
+            got = [s.phi(), s.psi()]
+            if precision == FP32:
+                s.solve_refined(100, 1e-5, 1e-4, 20)
+                got += [s.phi(), s.psi()]
+            ref.append(got)
+    mem = members()
+    with SweepBatch(mem) as b:
+        b.set_concurrent(chains)
+        b.solve_krylov(200, 1e-9 if precision == FP64 else 1e-5, 20)
+        b.sweep_step()
+        b.synchronize()
+        got = [[s.phi(), s.psi()] for s in mem]
+        if precision == FP32:
+            b.solve_refined(100, 1e-5, 1e-4, 20)
+            for g, s in zip(got, mem):
+                g += [s.phi(), s.psi()]
+    for g, r in zip(got, ref):
+        for a, c in zip(g, r):
+            assert np.array_equal(a, c)
+    for s in mem:
+        s.close()

@@ -300,6 +300,23 @@ bool angle_form(const t2_sweeper *s)
            s->use_graph;
 }
 
+t2::AngleSweep angle_tables(const t2_sweeper *s)
+{
+    t2::AngleSweep t{};
+    t.round_off = s->d_angles;
+    t.rounds = s->d_rounds;
+    t.order = s->d_angles + s->na + 1;
+    t.items = s->d_slot_items;
+    t.lag_off = s->sched.lagged.empty() ? nullptr
+                                        : s->d_angles + 2 * s->na + 1;
+    t.n_slots = int(s->angle_slots);
+    t.zero = int(s->angle_slots + s->angle_lag);
+    t.n_angles = int(s->na);
+    t.groups = int(s->ng);
+    t.chunks = int(s->ng) / s->angle_gc;
+    return t;
+}
+
 // psi_out = L^-1 (src + ang + ang_t).  Lagged faces read a snapshot of the
 // handle's psi taken before the sweep; a sweep into another buffer (the
 // refined solve's correction, whose previous value is zero) reads zeros
@@ -345,18 +362,8 @@ int enqueue_sweep(t2_sweeper *s, const double *ang, const void *ang_t,
         a.geo = geo;
         a.topo = s->d_item_topo;
         a.n_items = s->nc * s->na;
-        t2::AngleSweep t{};
-        t.round_off = s->d_angles;
-        t.rounds = s->d_rounds;
-        t.order = s->d_angles + s->na + 1;
-        t.items = s->d_slot_items;
-        t.lag_off = n_lag > 0 ? s->d_angles + 2 * s->na + 1 : nullptr;
-        t.n_slots = int(s->angle_slots);
-        t.zero = int(s->angle_slots + s->angle_lag);
-        t.n_angles = int(s->na);
-        t.groups = int(s->ng);
-        t.chunks = int(s->ng) / s->angle_gc;
-        T2_HIP(t2::launch_angle_sweep<T>(a, t, s->angle_block, s->stream));
+        T2_HIP(t2::launch_angle_sweep<T>(a, angle_tables(s), s->angle_block,
+                                         s->stream));
         return T2_OK;
     }
     const int64_t nb = int64_t(s->sched.batch_steps.size()) - 1;
@@ -2283,6 +2290,17 @@ struct t2_batch {
     // level form (built on first use)
     bool levels_built = false;
     std::vector<LevelGroup> groups;
+    // members swept with one block per angle, in up to two launches (by the
+    // LDS their blocks need)
+    std::vector<int> angle_idx;          // member of each table entry
+    void *d_angle_problems = nullptr;    // AngleProblem<T>
+    int2 *d_angle_runs = nullptr;
+    int32_t *d_angle_active = nullptr;   // active flags in table order
+    struct AngleLaunch {
+        int first_run, n_runs, n_blocks;
+        size_t lds;
+    };
+    std::vector<AngleLaunch> angle_launches;
     // queue form (built on first use)
     int64_t n_chunks = -1, grid = 0;
     void *d_problems = nullptr;
@@ -2293,13 +2311,12 @@ struct t2_batch {
     int32_t *d_active = nullptr;         // members swept by the next sweep
     std::vector<int32_t> active;         // host copy (kept alive for copies)
     std::vector<int32_t> uploaded;       // flags the device holds
-    hipGraphExec_t graph = nullptr;
+    // captured sweeps: [correction sweep][angle-dependent sources]
+    hipGraphExec_t graph[2][2] = {};
     // correction sweeps of the refined solve: each member's sweep writes its
     // residual buffer in place (its angle-dependent source) and lagged faces
-    // read zero; the tables point there while corr is set, and the sweep is
-    // captured in a graph of its own
+    // read zero; the tables point there while corr is set
     bool corr = false;
-    hipGraphExec_t graph_corr = nullptr;
     std::vector<std::vector<const void *>> snap;  // members' buffers
 };
 
@@ -2309,6 +2326,7 @@ std::vector<const void *> member_buffers(const t2_sweeper *m)
 {
     return {m->d_item_geo, m->d_item_topo, m->d_psi, m->d_src, m->d_lag_buf,
             m->d_lag_key, m->d_sigt, m->d_qang, m->d_pending, m->d_down,
+            m->d_slot_items, m->d_rounds, m->d_angles,
             reinterpret_cast<const void *>(intptr_t(m->sched.n_steps))};
 }
 
@@ -2354,6 +2372,15 @@ void free_levels(t2_batch *b)
             (void)hipFree(g.d_desc);
     }
     b->groups.clear();
+    for (void *p : {b->d_angle_problems, static_cast<void *>(b->d_angle_runs),
+                    static_cast<void *>(b->d_angle_active)})
+        if (p)
+            (void)hipFree(p);
+    b->d_angle_problems = nullptr;
+    b->d_angle_runs = nullptr;
+    b->d_angle_active = nullptr;
+    b->angle_idx.clear();
+    b->angle_launches.clear();
     b->levels_built = false;
 }
 
@@ -2370,12 +2397,12 @@ void free_batch_queue(t2_batch *b)
 
 void drop_batch_graph(t2_batch *b)
 {
-    if (b->graph)
-        (void)hipGraphExecDestroy(b->graph);
-    if (b->graph_corr)
-        (void)hipGraphExecDestroy(b->graph_corr);
-    b->graph = nullptr;
-    b->graph_corr = nullptr;
+    for (auto &row : b->graph)
+        for (hipGraphExec_t &g : row) {
+            if (g)
+                (void)hipGraphExecDestroy(g);
+            g = nullptr;
+        }
 }
 
 // Angular flux a member's batched sweep writes.
@@ -2422,6 +2449,13 @@ t2::BatchProblem<T> batch_problem(const t2_sweeper *m, const void *ang_t,
     return bp;
 }
 
+template <typename T>
+t2::AngleProblem<T> angle_problem(const t2_sweeper *m, const void *ang_t,
+                                  void *psi_out)
+{
+    return {batch_problem<T>(m, ang_t, psi_out).a, angle_tables(m)};
+}
+
 // Rewrites the device problem tables that exist (after a change of the
 // members' angle-dependent sources); the captured sweeps read them.
 template <typename T>
@@ -2437,6 +2471,17 @@ int write_tables(t2_batch *b)
                 member_psi_out(b, b->members[g.idx[j]]));
         T2_HIP(hipMemcpy(g.d_desc, desc.data(),
                          sizeof(t2::ProblemDesc<T>) * desc.size(),
+                         hipMemcpyHostToDevice));
+    }
+    if (b->d_angle_problems) {
+        std::vector<t2::AngleProblem<T>> probs(b->angle_idx.size());
+        for (size_t j = 0; j < probs.size(); j++) {
+            const t2_sweeper *m = b->members[b->angle_idx[j]];
+            probs[j] = angle_problem<T>(m, b->ang_t[b->angle_idx[j]],
+                                        member_psi_out(b, m));
+        }
+        T2_HIP(hipMemcpy(b->d_angle_problems, probs.data(),
+                         sizeof(t2::AngleProblem<T>) * probs.size(),
                          hipMemcpyHostToDevice));
     }
     if (b->d_problems) {
@@ -2532,12 +2577,78 @@ int build_level_group(t2_batch *b, LevelGroup &g)
     return T2_OK;
 }
 
+// One-block-per-angle members: their problem table and launches.  Blocks of
+// half the LDS or less run two a CU, the others one: a launch each, the
+// blocks with the most rounds first.
+template <typename T>
+int build_angle_batch(t2_batch *b)
+{
+    struct Part {
+        int member, blocks;
+        size_t lds;
+        double rounds;                   // of an average block
+    };
+    std::vector<Part> parts;
+    for (size_t i = 0; i < b->members.size(); i++) {
+        const t2_sweeper *m = b->members[i];
+        if (m->angle_gc <= 0)
+            continue;
+        const t2::AngleSweep t = angle_tables(m);
+        if (!t2::angle_sweep_valid(
+                batch_problem<T>(m, b->ang_t[i], member_psi_out(b, m)).a, t))
+            return fail(T2_ERR_STATE, "batch member's sweep tables");
+        parts.push_back({int(i), t2::angle_blocks(t),
+                         t2::angle_lds_bytes(t.zero + 1, m->angle_gc,
+                                             sizeof(T)),
+                         double(m->n_rounds) / double(m->na)});
+    }
+    if (parts.empty())
+        return T2_OK;
+    auto big = [](const Part &p) { return p.lds > t2::kMaxLds / 2; };
+    std::stable_sort(parts.begin(), parts.end(),
+                     [&](const Part &x, const Part &y) {
+                         return big(x) != big(y) ? big(x)
+                                                 : x.rounds > y.rounds;
+                     });
+    std::vector<t2::AngleProblem<T>> probs;
+    std::vector<int2> runs;
+    for (const Part &p : parts) {
+        const t2_sweeper *m = b->members[p.member];
+        if (b->angle_launches.empty() ||
+            big(p) != (b->angle_launches.back().lds > t2::kMaxLds / 2))
+            b->angle_launches.push_back({int(runs.size()), 0, 0, 0});
+        t2_batch::AngleLaunch &l = b->angle_launches.back();
+        runs.push_back(make_int2(l.n_blocks, int(probs.size())));
+        l.n_runs++;
+        l.n_blocks += p.blocks;
+        l.lds = std::max(l.lds, p.lds);
+        probs.push_back(angle_problem<T>(m, b->ang_t[p.member],
+                                         member_psi_out(b, m)));
+        b->angle_idx.push_back(p.member);
+    }
+    T2_HIP(hipMalloc(&b->d_angle_problems,
+                     sizeof(t2::AngleProblem<T>) * probs.size()));
+    T2_HIP(hipMalloc(reinterpret_cast<void **>(&b->d_angle_runs),
+                     sizeof(int2) * runs.size()));
+    T2_HIP(hipMalloc(reinterpret_cast<void **>(&b->d_angle_active),
+                     sizeof(int32_t) * probs.size()));
+    T2_HIP(hipMemcpy(b->d_angle_problems, probs.data(),
+                     sizeof(t2::AngleProblem<T>) * probs.size(),
+                     hipMemcpyHostToDevice));
+    T2_HIP(hipMemcpy(b->d_angle_runs, runs.data(), sizeof(int2) * runs.size(),
+                     hipMemcpyHostToDevice));
+    return T2_OK;
+}
+
 int build_levels(t2_batch *b)
 {
     free_levels(b);
+    T2_TRY(b->precision == T2_FP64 ? build_angle_batch<double>(b)
+                                   : build_angle_batch<float>(b));
     std::vector<int> ngs;
     for (auto *m : b->members)
-        if (std::find(ngs.begin(), ngs.end(), int(m->ng)) == ngs.end())
+        if (m->angle_gc <= 0 &&
+            std::find(ngs.begin(), ngs.end(), int(m->ng)) == ngs.end())
             ngs.push_back(int(m->ng));
     std::sort(ngs.begin(), ngs.end());
     // one merged schedule per group count, or, for parallel chains, up to
@@ -2547,7 +2658,7 @@ int build_levels(t2_batch *b)
     for (int ng : ngs) {
         std::vector<int> idx;
         for (size_t i = 0; i < b->members.size(); i++)
-            if (b->members[i]->ng == ng)
+            if (b->members[i]->angle_gc <= 0 && b->members[i]->ng == ng)
                 idx.push_back(int(i));
         auto work = [&](int i) {
             return b->members[i]->nc * b->members[i]->na * b->members[i]->ng;
@@ -2668,6 +2779,15 @@ int batch_enqueue(t2_batch *b)
             b->d_chunks, q, b->grid, b->stream));
         return T2_OK;
     }
+    // all members carry an angle-dependent source or none does
+    auto launch_angles = [&]() {
+        for (const auto &l : b->angle_launches)
+            T2_HIP(t2::launch_angle_batch<T>(
+                static_cast<const t2::AngleProblem<T> *>(b->d_angle_problems),
+                b->d_angle_runs + l.first_run, l.n_runs, l.n_blocks,
+                b->d_angle_active, b->ang_t[0] != nullptr, l.lds, b->stream));
+        return T2_OK;
+    };
     auto launch = [&](LevelGroup &g, int64_t st, hipStream_t stream) {
         t2::SweepArgs<T> a{};
         a.problems = static_cast<const t2::ProblemDesc<T> *>(g.d_desc);
@@ -2679,25 +2799,33 @@ int batch_enqueue(t2_batch *b)
         return T2_OK;
     };
     const size_t ng = b->groups.size();
-    if (b->concurrent > 0 && ng > 1) {
-        // merged schedules share nothing: group g > 0 runs its merged steps
-        // on a stream of its own (a parallel branch of the captured graph),
-        // forked from and joined to the batch's
+    const size_t main_group = b->angle_launches.empty() ? 1 : 0;
+    if (b->concurrent > 0 && ng > main_group) {
+        // merged schedules share nothing: they run on streams of their own
+        // (parallel branches of the captured graph), forked from and joined
+        // to the batch's, which takes the one-block-per-angle launches or,
+        // without any, the first schedule
         T2_HIP(hipEventRecord(b->fork_ev, b->stream));
-        for (size_t i = 1; i < ng; i++) {
+        for (size_t i = main_group; i < ng; i++) {
             LevelGroup &g = b->groups[i];
-            T2_HIP(hipStreamWaitEvent(b->side[i - 1], b->fork_ev, 0));
+            const size_t k = i - main_group;
+            T2_HIP(hipStreamWaitEvent(b->side[k], b->fork_ev, 0));
             for (int64_t st = 0; st + 1 < int64_t(g.step_off.size()); st++)
-                T2_TRY(launch(g, st, b->side[i - 1]));
-            T2_HIP(hipEventRecord(b->join_ev[i - 1], b->side[i - 1]));
+                T2_TRY(launch(g, st, b->side[k]));
+            T2_HIP(hipEventRecord(b->join_ev[k], b->side[k]));
         }
-        LevelGroup &g0 = b->groups[0];
-        for (int64_t st = 0; st + 1 < int64_t(g0.step_off.size()); st++)
-            T2_TRY(launch(g0, st, b->stream));
-        for (size_t i = 1; i < ng; i++)
-            T2_HIP(hipStreamWaitEvent(b->stream, b->join_ev[i - 1], 0));
+        T2_TRY(launch_angles());
+        if (main_group == 1) {
+            LevelGroup &g0 = b->groups[0];
+            for (int64_t st = 0; st + 1 < int64_t(g0.step_off.size()); st++)
+                T2_TRY(launch(g0, st, b->stream));
+        }
+        for (size_t i = main_group; i < ng; i++)
+            T2_HIP(hipStreamWaitEvent(b->stream, b->join_ev[i - main_group],
+                                      0));
         return T2_OK;
     }
+    T2_TRY(launch_angles());
     int64_t longest = 0;
     for (auto &g : b->groups)
         longest = std::max<int64_t>(longest, int64_t(g.step_off.size()) - 1);
@@ -2780,6 +2908,15 @@ int batch_sweep(t2_batch *b)
                                   hipMemcpyHostToDevice, b->stream));
             T2_HIP(hipStreamSynchronize(b->stream));
         }
+        if (b->d_angle_active) {
+            std::vector<int32_t> ga(b->angle_idx.size());
+            for (size_t j = 0; j < ga.size(); j++)
+                ga[j] = b->active[b->angle_idx[j]];
+            T2_HIP(hipMemcpyAsync(b->d_angle_active, ga.data(),
+                                  sizeof(int32_t) * ga.size(),
+                                  hipMemcpyHostToDevice, b->stream));
+            T2_HIP(hipStreamSynchronize(b->stream));
+        }
         T2_HIP(hipStreamSynchronize(b->stream));
         b->uploaded = b->active;
     }
@@ -2788,7 +2925,8 @@ int batch_sweep(t2_batch *b)
         if (!b->fork_ev)
             T2_HIP(hipEventCreateWithFlags(&b->fork_ev,
                                            hipEventDisableTiming));
-        while (b->side.size() + 1 < b->groups.size()) {
+        while (b->side.size() + 1 <
+               b->groups.size() + (b->angle_launches.empty() ? 0 : 1)) {
             hipStream_t st = nullptr;
             hipEvent_t ev = nullptr;
             T2_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
@@ -2797,7 +2935,7 @@ int batch_sweep(t2_batch *b)
             b->join_ev.push_back(ev);
         }
     }
-    hipGraphExec_t &exec = b->corr ? b->graph_corr : b->graph;
+    hipGraphExec_t &exec = b->graph[b->corr][b->ang_t[0] != nullptr];
     if (!exec) {
         hipGraph_t g = nullptr;
         T2_HIP(hipStreamBeginCapture(b->stream,

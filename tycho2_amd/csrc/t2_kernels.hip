@@ -786,13 +786,15 @@ __device__ __forceinline__ void buffer_geo(Rsrc r, uint32_t off,
 // ROW: one group in all, so that a cell's four values are contiguous and move
 // in one access.
 template <typename T, int GC, int ANG, bool ROW>
-__global__ void __launch_bounds__(kMaxAngleBlock)
-angle_sweep_kernel(const SweepArgs<T> p, const AngleSweep t)
+__device__ __forceinline__ void sweep_angle(const SweepArgs<T> &p,
+                                            const AngleSweep &t, int task,
+                                            char *lds_raw)
 {
-    extern __shared__ char lds_raw[];
     int32_t *const done = reinterpret_cast<int32_t *>(lds_raw);
     T *const live = reinterpret_cast<T *>(lds_raw + kAngleLdsHead);
-    const int x = int(blockIdx.x % kXcds), j = int(blockIdx.x / kXcds);
+    // the chunks of an angle run on one XCD (blocks go round robin), which
+    // completes the cache lines they share in its L2
+    const int x = task % kXcds, j = task / kXcds;
     const int ai = (j / t.chunks) * kXcds + x;
     if (ai >= t.n_angles)
         return;
@@ -997,6 +999,49 @@ angle_sweep_kernel(const SweepArgs<T> p, const AngleSweep t)
         }
         if constexpr (!kEarly)
             load_inputs(r0, rec0, in);
+    }
+}
+
+template <typename T, int GC, int ANG, bool ROW>
+__global__ void __launch_bounds__(kMaxAngleBlock)
+angle_sweep_kernel(const SweepArgs<T> p, const AngleSweep t)
+{
+    extern __shared__ char lds_raw[];
+    sweep_angle<T, GC, ANG, ROW>(p, t, int(blockIdx.x), lds_raw);
+}
+
+// Several problems in one launch: each run of blocks sweeps one problem (its
+// first block a multiple of kXcds), whose groups per block select the form.
+// Merged step launches gave a small member's levels a share of one launch,
+// but every level of the deepest member its 4 us; here each block runs at its
+// own pace.  Six problems of 2,058 to 24,576 cells, 32 to 288 angles and 1 to
+// 32 groups, FP64 GMRES in lock step: 82.1 -> 31.4 ms a solve.  Blocks of 512
+// threads, two a CU within 128 registers.
+template <typename T, int ANG>
+__global__ void __launch_bounds__(kBatchAngleBlock, 4)
+angle_batch_kernel(const AngleProblem<T> *problems, const int2 *runs,
+                   int n_runs, const int32_t *active)
+{
+    extern __shared__ char lds_raw[];
+    int r = 0;
+    while (r + 1 < n_runs && runs[r + 1].x <= int(blockIdx.x))
+        r++;
+    const int2 run = runs[r];
+    if (!active[run.y])
+        return;
+    const AngleProblem<T> &ap = problems[run.y];
+    const int task = int(blockIdx.x) - run.x;
+    switch (ap.t.groups / ap.t.chunks) {
+    case 1:
+        if (ap.t.groups == 1)
+            sweep_angle<T, 1, ANG, true>(ap.a, ap.t, task, lds_raw);
+        else
+            sweep_angle<T, 1, ANG, false>(ap.a, ap.t, task, lds_raw);
+        break;
+    case 2: sweep_angle<T, 2, ANG, false>(ap.a, ap.t, task, lds_raw); break;
+    case 4: sweep_angle<T, 4, ANG, false>(ap.a, ap.t, task, lds_raw); break;
+    case 8: sweep_angle<T, 8, ANG, false>(ap.a, ap.t, task, lds_raw); break;
+    default: break;
     }
 }
 
@@ -1743,10 +1788,9 @@ hipError_t launch_angle_k(const SweepArgs<T> &args, const AngleSweep &t,
         hipFuncAttributeMaxDynamicSharedMemorySize, int(kMaxLds));
     if (e != hipSuccess)
         return e;
-    const unsigned grid =
-        unsigned((t.n_angles + kXcds - 1) / kXcds * kXcds * t.chunks);
-    hipLaunchKernelGGL((angle_sweep_kernel<T, GC, ANG, ROW>), dim3(grid),
-                       dim3(block), lds, stream, args, t);
+    hipLaunchKernelGGL((angle_sweep_kernel<T, GC, ANG, ROW>),
+                       dim3(unsigned(angle_blocks(t))), dim3(block), lds,
+                       stream, args, t);
     return hipGetLastError();
 }
 
@@ -1762,20 +1806,32 @@ hipError_t launch_angle_g(const SweepArgs<T> &args, const AngleSweep &t,
     return launch_angle_k<T, GC, 0, ROW>(args, t, block, lds, stream);
 }
 
+// What the kernels assume of a sweep's tables.
+template <typename T>
+bool angle_sweep_valid(const SweepArgs<T> &args, const AngleSweep &t)
+{
+    const int gc = t.chunks > 0 ? t.groups / t.chunks : 0;
+    // byte offsets within a plane are 32-bit, below kOutside
+    const int64_t plane = args.nc * 4 * t.groups * int64_t(sizeof(double));
+    return (gc == 1 || gc == 2 || gc == 4 || gc == 8) &&
+           gc * t.chunks == t.groups && t.n_angles > 0 &&
+           t.zero < kMaxSlots &&
+           angle_lds_bytes(t.zero + 1, gc, sizeof(T)) <= kMaxLds &&
+           plane < (int64_t(1) << 32) && args.solver == kSolveNoPivot &&
+           !args.problems && !args.active &&
+           !(args.src_ang && args.src_ang_t) &&
+           !(sizeof(T) == 8 && args.src_ang_t);
+}
+
 template <typename T>
 hipError_t launch_angle_sweep(const SweepArgs<T> &args, const AngleSweep &t,
                               int block, hipStream_t stream)
 {
-    const int gc = t.chunks > 0 ? t.groups / t.chunks : 0;
-    const size_t lds = angle_lds_bytes(t.zero + 1, gc, sizeof(T));
-    // the kernel's byte offsets within a plane are 32-bit, below kOutside
-    const int64_t plane = args.nc * 4 * t.groups * int64_t(sizeof(double));
-    if (block < 64 || block > kMaxAngleBlock || block % 64 || lds > kMaxLds ||
-        gc * t.chunks != t.groups || t.n_angles <= 0 || t.zero >= kMaxSlots ||
-        plane >= (int64_t(1) << 32) || args.solver != kSolveNoPivot ||
-        args.problems || args.active || (args.src_ang && args.src_ang_t) ||
-        (sizeof(T) == 8 && args.src_ang_t))
+    if (block < 64 || block > kMaxAngleBlock || block % 64 ||
+        !angle_sweep_valid(args, t))
         return hipErrorInvalidValue;
+    const int gc = t.groups / t.chunks;
+    const size_t lds = angle_lds_bytes(t.zero + 1, gc, sizeof(T));
     switch (gc) {
     case 1:
         return t.groups == 1
@@ -1786,6 +1842,33 @@ hipError_t launch_angle_sweep(const SweepArgs<T> &args, const AngleSweep &t,
     case 8: return launch_angle_g<T, 8, false>(args, t, block, lds, stream);
     default: return hipErrorInvalidValue;
     }
+}
+
+template <typename T>
+hipError_t launch_angle_batch(const AngleProblem<T> *problems,
+                              const int2 *runs, int n_runs, int n_blocks,
+                              const int32_t *active, bool ang_t, size_t lds,
+                              hipStream_t stream)
+{
+    if (n_runs <= 0)
+        return hipSuccess;
+    if (lds > kMaxLds || (ang_t && sizeof(T) == 8))
+        return hipErrorInvalidValue;
+    auto go = [&](auto kernel) {
+        const hipError_t e = hipFuncSetAttribute(
+            reinterpret_cast<const void *>(kernel),
+            hipFuncAttributeMaxDynamicSharedMemorySize, int(kMaxLds));
+        if (e != hipSuccess)
+            return e;
+        hipLaunchKernelGGL(kernel, dim3(unsigned(n_blocks)),
+                           dim3(kBatchAngleBlock), lds, stream, problems, runs,
+                           n_runs, active);
+        return hipGetLastError();
+    };
+    if constexpr (sizeof(T) == 4)
+        if (ang_t)
+            return go(&angle_batch_kernel<T, 2>);
+    return go(&angle_batch_kernel<T, 0>);
 }
 
 hipError_t launch_slot_items(const ItemTopo *topo, const uint16_t *slot,
@@ -2113,6 +2196,12 @@ hipError_t launch_fill(double *x, double v, int64_t n, hipStream_t stream)
                                              int, hipStream_t);               \
     template hipError_t launch_angle_sweep<T>(const SweepArgs<T> &,           \
                                               const AngleSweep &, int,        \
+                                              hipStream_t);                   \
+    template bool angle_sweep_valid<T>(const SweepArgs<T> &,                  \
+                                       const AngleSweep &);                   \
+    template hipError_t launch_angle_batch<T>(const AngleProblem<T> *,        \
+                                              const int2 *, int, int,         \
+                                              const int32_t *, bool, size_t,  \
                                               hipStream_t);                   \
     template hipError_t launch_residual<T>(const ResidualArgs<T> &, int,      \
                                            hipStream_t);                      \

@@ -182,6 +182,29 @@ inline size_t angle_lds_bytes(int64_t slots, int gc, size_t value)
 template <typename T>
 hipError_t launch_angle_sweep(const SweepArgs<T> &args, const AngleSweep &t,
                               int block, hipStream_t stream);
+// Blocks of a sweep: a multiple of 8 (one XCD per angle's chunks).
+inline int angle_blocks(const AngleSweep &t)
+{
+    return (t.n_angles + 7) / 8 * 8 * t.chunks;
+}
+template <typename T>
+bool angle_sweep_valid(const SweepArgs<T> &args, const AngleSweep &t);
+
+// Several problems in one launch.  runs: {first block, problem}, ascending;
+// problems whose active flag is 0 are skipped; ang_t: every problem carries
+// an angle-dependent source in T.
+constexpr int kBatchAngleBlock = 512;
+template <typename T>
+struct AngleProblem {
+    SweepArgs<T> a;
+    AngleSweep t;
+};
+template <typename T>
+hipError_t launch_angle_batch(const AngleProblem<T> *problems,
+                              const int2 *runs, int n_runs, int n_blocks,
+                              const int32_t *active, bool ang_t, size_t lds,
+                              hipStream_t stream);
+
 hipError_t launch_slot_items(const ItemTopo *topo, const uint16_t *slot,
                              const int32_t *lag_off, int n_slots, int zero,
                              int64_t n, int64_t nc, SlotItem *out,
