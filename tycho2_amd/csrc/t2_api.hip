@@ -317,6 +317,22 @@ t2::AngleSweep angle_tables(const t2_sweeper *s)
     return t;
 }
 
+// Step launches store psi past the caches when an average step writes more
+// of it than kCachedStep: a step reads about three times what it writes, and
+// its cells are read for a few steps after it, so beyond about a sixteenth of
+// the 256 MB last-level cache plain stores only displace the inputs.
+// Streamed / plain, ms a pass: 73,002 cells x 128 angles x 16 groups FP32
+// (7.5 MB a step) 2.82 / 2.56; 93,750 x 72 x 32 FP64 (3 MB) 12.5 / 12.0;
+// 384,000 x 128 x 16 FP32 (22 MB) 11.42 / 11.51, FP64 (45 MB) 20.7 / 21.0;
+// 1,296,000 x 128 x 16 FP64 (98 MB) 56.4 / 57.3.
+constexpr double kCachedStep = 16e6;
+
+bool stream_psi(int64_t items, int64_t groups, size_t value, int64_t steps)
+{
+    return double(items) * 4.0 * double(groups) * double(value) >
+           kCachedStep * double(std::max<int64_t>(1, steps));
+}
+
 // psi_out = L^-1 (src + ang + ang_t).  Lagged faces read a snapshot of the
 // handle's psi taken before the sweep; a sweep into another buffer (the
 // refined solve's correction, whose previous value is zero) reads zeros
@@ -346,6 +362,8 @@ int enqueue_sweep(t2_sweeper *s, const double *ang, const void *ang_t,
     a.lag_buf = static_cast<const T *>(s->d_lag_buf);
     a.solver = cell_solver(s->gauss);
     a.items_per_lane = s->ipl;
+    a.stream_psi = stream_psi(s->nc * s->na, s->ng, sizeof(T),
+                              s->sched.n_steps);
     const auto *geo = static_cast<const t2::ItemGeo<T> *>(s->d_item_geo);
     auto launch_steps = [&](int64_t lo, int64_t hi, hipStream_t stream) {
         for (int64_t st = lo; st < hi; st++) {
@@ -2795,6 +2813,8 @@ int batch_enqueue(t2_batch *b)
         a.geo = static_cast<const t2::ItemGeo<T> *>(g.d_geo) + g.step_off[st];
         a.topo = g.d_topo + g.step_off[st];
         a.n_items = g.step_off[st + 1] - g.step_off[st];
+        a.stream_psi = stream_psi(g.n_items, g.ng, sizeof(T),
+                                  int64_t(g.step_off.size()) - 1);
         T2_HIP(t2::launch_sweep_step<T>(a, g.ng, 1, b->block, stream));
         return T2_OK;
     };

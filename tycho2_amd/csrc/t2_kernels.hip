@@ -260,9 +260,11 @@ __global__ void build_items_kernel(const uint32_t *__restrict__ work,
 // gl: gl, gl + LPI, ... (LPI = G / GPL lanes per item).  COH: upwind psi is
 // read and psi written at the device coherence point (sc1 loads, write-
 // through stores), as the ready-queue kernel needs; otherwise plain cached
-// accesses (kernel boundaries order the per-step launches).
+// accesses (kernel boundaries order the per-step launches).  STREAM: psi is
+// stored past the caches (SweepArgs::stream_psi; a compile-time choice,
+// because a branch at the stores costs 1% of a sweep).
 template <typename T, int G, int GPL, bool COH = false,
-          int SOLVER = kSolveNoPivot>
+          int SOLVER = kSolveNoPivot, bool STREAM = true>
 __device__ __forceinline__ void solve_item(const SweepArgs<T> &p,
                                            int64_t item, int gl,
                                            const ItemTopo &t)
@@ -388,18 +390,25 @@ __device__ __forceinline__ void solve_item(const SweepArgs<T> &p,
             solve_nopivot<T>(m, b);
 
         T *dst = psi + size_t(t.angle) * plane + own + g;
+        if constexpr (COH) {
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            if constexpr (COH)
+            for (int v = 0; v < 4; v++)
                 __hip_atomic_store(dst + v * G, b[v], __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
-            else  // streamed: keeps psi from evicting cached inputs
-                __builtin_nontemporal_store(b[v], dst + v * G);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                if constexpr (STREAM)
+                    __builtin_nontemporal_store(b[v], dst + v * G);
+                else
+                    dst[v * G] = b[v];
+            }
         }
     }
 }
 
-template <typename T, int G, int GPL, int SOLVER = kSolveNoPivot>
+template <typename T, int G, int GPL, int SOLVER = kSolveNoPivot,
+          bool STREAM = true>
 __global__ void __launch_bounds__(kMaxBlock)
 sweep_step_kernel(const SweepArgs<T> p)
 {
@@ -418,7 +427,7 @@ sweep_step_kernel(const SweepArgs<T> p)
     const ItemTopo t = p.topo[item];
     if (p.active && !p.active[t.problem])
         return;
-    solve_item<T, G, GPL, false, SOLVER>(p, item, gl, t);
+    solve_item<T, G, GPL, false, SOLVER, STREAM>(p, item, gl, t);
 }
 
 // ------------------------------------------------------- two items per lane
@@ -1363,8 +1372,13 @@ hipError_t launch_g(const SweepArgs<T> &args, int gpl, int block,
     }
     switch (gpl) {
     case 1:
-        hipLaunchKernelGGL((sweep_step_kernel<T, G, 1>), dim3(grid),
-                           dim3(block), 0, stream, args);
+        if (args.stream_psi)
+            hipLaunchKernelGGL((sweep_step_kernel<T, G, 1>), dim3(grid),
+                               dim3(block), 0, stream, args);
+        else
+            hipLaunchKernelGGL(
+                (sweep_step_kernel<T, G, 1, kSolveNoPivot, false>), dim3(grid),
+                dim3(block), 0, stream, args);
         break;
     case 2:
         if constexpr (G >= 2) {

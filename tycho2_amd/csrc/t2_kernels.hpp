@@ -83,6 +83,9 @@ struct SweepArgs {
     // CellSolver; the level engine's kernels take any, the ready-queue
     // kernels kSolveNoPivot
     int solver;
+    // step launches, one group and item per lane, kSolveNoPivot: psi stored
+    // past the caches (always so with the other launch shapes and solvers)
+    bool stream_psi;
     // level engine, kSolveNoPivot, one group per lane, one problem (no
     // problems / active tables): 2 solves two items per lane, their loads
     // issued before either solve (0 or 1: one item per lane)
