@@ -111,3 +111,27 @@ def test_batch_of_both_forms(precision, chains):
             assert np.array_equal(a, c)
     for s in mem:
         s.close()
+
+
+def test_levels_after_lagging(monkeypatch):
+    """Angles at 45 degrees: the schedule levels the graph left after lagging
+    (far fewer steps than the stalling traversal's levels), and step launches
+    over it still give the oracle's sweep."""
+    import oracle as orc
+    from tycho2_amd.sweeper import mesh_geometry, sweep_levels
+    print("levels after lagging", flush=True)
+    monkeypatch.setenv("T2_NO_GRAPH", "1")
+    sm = meshmod.kuhn_cube(6, 0.15, seed=7)
+    conn = meshmod.tycho_connectivity(sm)
+    omega, wt = product_quadrature(6)
+    _, area, normal = mesh_geometry(sm, conn)
+    levels, n_lag = sweep_levels(conn.adj_cell, area, normal, omega)
+    rng = np.random.default_rng(3)
+    st = rng.uniform(0.5, 2.0, (sm.n_cells, 2))
+    src = rng.uniform(0.0, 1.0, (sm.n_cells, omega.shape[0], 4, 2))
+    with SweeperHIP(sm, conn, omega, wt, 2, st, 0.5 * st, FP64) as s:
+        assert s.info()["n_lagged"] == n_lag > 0
+        assert s.info()["n_steps"] < (levels.max() + 1) // 2
+        psi = s.sweep(np.zeros_like(src), src)
+    ref, _ = orc.sweep(orc.build_mesh(sm), omega, 2, st, src)
+    assert np.abs(psi - ref).max() <= 1e-12 * np.abs(ref).max()
