@@ -854,11 +854,19 @@ __device__ __forceinline__ void sweep_angle(const SweepArgs<T> &p,
         T sig, q[4];
         std::conditional_t<ANG == 1, double, T> qa[4];
     };
+    // a round's entry, issued now and made scalar where it is first used (the
+    // buffer descriptors below have to be)
     auto round_at = [&](int i) {
         AngleRound r{0, 0, 0};
         if (i < n_rounds)
             r = rounds[i];
         return r;
+    };
+    auto uniform = [](const AngleRound &r) {
+        return AngleRound{
+            uint32_t(__builtin_amdgcn_readfirstlane(int(r.item))),
+            uint32_t(__builtin_amdgcn_readfirstlane(int(r.count))),
+            uint32_t(__builtin_amdgcn_readfirstlane(int(r.need)))};
     };
     auto load_record = [&](const AngleRound &r) {
         const Rsrc b = buffer_of(t.items + r.item,
@@ -909,13 +917,16 @@ __device__ __forceinline__ void sweep_angle(const SweepArgs<T> &p,
     // (128 registers for 16 wavefronts a block), and skipping the faces that
     // no lane reads pays for its branch
     constexpr bool kEarly = sizeof(T) == 4;
-    AngleRound r0 = round_at(k), r1 = round_at(k + n_waves);
+    AngleRound r0 = uniform(round_at(k));
+    AngleRound r1 = uniform(round_at(k + n_waves));
+    AngleRound r2 = round_at(k + 2 * n_waves);
     Record rec0 = load_record(r0), rec1 = load_record(r1);
     Inputs in;
     load_inputs(r0, rec0, in);
     for (; k < n_rounds; k += n_waves) {
         // ahead of the earlier levels: this round's factors and LDS
-        // addresses, the next one's inputs, the record of the one after it
+        // addresses, the next one's inputs, the record of the one after it,
+        // the entry of the third
         T a12[4], q[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -947,11 +958,12 @@ __device__ __forceinline__ void sweep_angle(const SweepArgs<T> &p,
             reads[kk] = kEarly || __any(mine && at[3 * kk] <
                                                     uint32_t(t.zero) * 4 * GC);
         r0 = r1;
-        r1 = round_at(k + 2 * n_waves);
+        r1 = uniform(r2);
         rec0 = rec1;
         if constexpr (kEarly)
             load_inputs(r0, rec0, in);
         rec1 = load_record(r1);
+        r2 = round_at(k + 3 * n_waves);
 
         uint32_t polls = 0;
         while (__builtin_amdgcn_readfirstlane(__hip_atomic_load(
@@ -1038,7 +1050,17 @@ angle_batch_kernel(const AngleProblem<T> *problems, const int2 *runs,
     const int2 run = runs[r];
     if (!active[run.y])
         return;
-    const AngleProblem<T> &ap = problems[run.y];
+    // the block's problem in scalar registers, as kernel arguments would be
+    // (a buffer descriptor built from vector registers costs a loop)
+    constexpr int kWords = sizeof(AngleProblem<T>) / sizeof(uint32_t);
+    struct Words {
+        uint32_t w[kWords];
+    } words;
+    const uint32_t *from = reinterpret_cast<const uint32_t *>(problems + run.y);
+#pragma unroll
+    for (int i = 0; i < kWords; i++)
+        words.w[i] = uint32_t(__builtin_amdgcn_readfirstlane(int(from[i])));
+    const AngleProblem<T> ap = __builtin_bit_cast(AngleProblem<T>, words);
     const int task = int(blockIdx.x) - run.x;
     switch (ap.t.groups / ap.t.chunks) {
     case 1:
