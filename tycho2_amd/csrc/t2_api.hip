@@ -886,37 +886,43 @@ void free_angle_form(t2_sweeper *s)
 }
 
 // Groups per block of the one-block-per-angle form, 0 if none will do.  The
-// table of `slots` slots has to fit the LDS, and a block's part of a vertex
-// row has to be the row or 16 bytes of it: with smaller parts the blocks of
-// an angle drift apart and psi's cache lines leave half written (93,750 cells
-// x 72 angles x 32 groups in FP64, one group a block: 18.4 ms a pass with
-// three handles at work against 8.2 ms by step launches).  Of those, the most
-// that leave kMinAngleBlocks blocks, because a block's records are read once
-// per gc groups (6,000 cells x 32 angles x 16 groups in FP64: 114, 121 and
-// 165 us a sweep with 256, 128 and 64 blocks).
+// table of `slots` slots has to fit the LDS.  A block's part of a vertex row
+// has to be the row, 16 bytes of it, or one of few parts (at most half as many
+// as it has bytes): many small parts drift apart and psi's cache lines leave
+// half written.  Step launches against that form, us a pass with three handles
+// at work: 93,750 cells x 72 angles x 32 groups FP64 in 32 parts of 8 bytes
+// 8,200 / 18,400; 162,000 x 128 x 4 FP32 in 2 parts of 8 bytes 2,797 / 2,288;
+// 93,750 x 32 x 4 FP64 in 4 of 8 bytes 668 / 547; 384,000 x 128 x 2 FP32 in 2
+// of 4 bytes 4,958 / 4,543.  Of those, the most groups that leave
+// kMinAngleBlocks blocks, because a block's records are read once per gc
+// groups (6,000 cells x 32 angles x 16 groups in FP64: 114, 121 and 165 us a
+// sweep with 256, 128 and 64 blocks).
 constexpr int64_t kMinAngleBlocks = 128;
 
 int angle_groups(const t2_sweeper *s, int64_t slots)
 {
     int gc = 0;
-    for (int c = 1; c <= 8 && c <= s->ng; c *= 2)
-        if ((c == s->ng || c * s->tsize() >= 16) &&
-            t2::angle_lds_bytes(slots, c, s->tsize()) <= t2::kMaxLds &&
+    for (int64_t c = 1; c <= 8 && c <= s->ng; c *= 2) {
+        const int64_t part = c * int64_t(s->tsize());
+        if ((c == s->ng || part >= 16 || s->ng / c <= part / 2) &&
+            t2::angle_lds_bytes(slots, int(c), s->tsize()) <= t2::kMaxLds &&
             (gc == 0 || s->na * (s->ng / c) >= kMinAngleBlocks))
-            gc = c;
+            gc = int(c);
+    }
     return gc;
 }
 
 // Whether that form is faster than the step launches: its bytes per solve
 // (records once per gc groups, source and psi) at the 3 TB/s it reaches
 // against 3.6 us per step and the step launches' 13.5 values per solve at
-// 5.2 TB/s.  Measured a sweep, angle form / step launches:
-//   750 cells,  32 angles, 1 group,  FP64    44 /   179 us
-//   20,250      72          1        FP32   922 /  5493 (1,703 steps)
-//   34,992     128          4        FP64   539 /  1471
-//   48,000     288          8        FP32  1897 /  2778
-//   73,002     128         16        FP32  3136 /  2819 (not taken: 2 groups)
+// 5.2 TB/s, more of them wasted the shorter a vertex row is than 32 bytes.
+// Measured a sweep, angle form / step launches (us):
+//   750 cells,  32 angles, 1 group,  FP64    34 /   179
+//   34,992     128          4        FP64   533 /  1471
+//   48,000     288          8        FP32  1875 /  2778
+//   73,002     128         16        FP32  3136 /  2560 (not taken)
 //   384,000    128          1        FP32  2760 /  5227
+//   196,608    128          4        FP64  4530 /  4450 (not taken)
 bool angle_pays(const t2_sweeper *s, int gc)
 {
     if (gc <= 0)
@@ -927,8 +933,10 @@ bool angle_pays(const t2_sweeper *s, int gc)
                                   ? sizeof(t2::ItemGeo<double>)
                                   : sizeof(t2::ItemGeo<float>));
     const double solves = double(s->nc) * double(s->na) * double(s->ng);
+    const double waste = std::max(1.0, 32.0 / (w * double(s->ng)));
     return solves * (rec / gc + 8.0 * w) / 3.0e12 <
-           3.6e-6 * double(s->sched.n_steps) + solves * 13.5 * w / 5.2e12;
+           3.6e-6 * double(s->sched.n_steps) +
+               solves * 13.5 * w * waste / 5.2e12;
 }
 
 // Tables of the one-block-per-angle form, where it applies (before the work
