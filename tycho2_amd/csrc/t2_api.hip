@@ -1194,7 +1194,7 @@ int setup_device(t2_sweeper *s, const double *weights, const double *sigma_s)
     T2_TRY(dalloc_t(s, &s->d_phi, sizeof(double) * n_phi));
     T2_TRY(dalloc_t(s, &s->d_phi_old, sizeof(double) * n_phi));
     T2_TRY(dalloc_t(s, &s->d_red, sizeof(double) * t2::kRedBlocks * 64));
-    T2_TRY(dalloc_t(s, &s->d_scal, sizeof(double) * 64));
+    T2_TRY(dalloc_t(s, &s->d_scal, sizeof(double) * t2::kArnoldiScalars));
     T2_TRY(zero_psi(s));
     T2_TRY(total_source(s, nullptr, nullptr));
     T2_HIP(t2::launch_fill(s->d_phi, 0.0, n_phi, s->stream));
@@ -1247,9 +1247,9 @@ struct Gmres {
     double *x = nullptr, *V = nullptr, *hist = nullptr;
     int64_t n = 0, m = 0, iter_max = 0, it = 0, j = 0;
     double bnorm = 0, target = 0, rnorm = 0;
-    bool x_zero = true;
+    bool x_zero = true, orthogonal = false;
     State state = kCycle;
-    std::vector<double> H, cs, sn, g, y, h, h2;
+    std::vector<double> H, cs, sn, g, y, h;
     const double *req_in = nullptr;
     double *req_out = nullptr;
 
@@ -1278,8 +1278,8 @@ struct Gmres {
         sn.assign(m, 0.0);
         g.assign(m + 1, 0.0);
         y.assign(m, 0.0);
-        h.assign(m + 1, 0.0);
-        h2.assign(m + 1, 0.0);
+        h.assign(t2::kArnoldiScalars, 0.0);
+        orthogonal = false;
         state = kCycle;
         return T2_OK;
     }
@@ -1301,6 +1301,19 @@ struct Gmres {
         T2_HIP(hipStreamSynchronize(s->stream));
         x_zero = false;
         state = kCycle;
+        return T2_OK;
+    }
+
+    // Enqueues the new vector's orthogonalisation once y = A v is enqueued;
+    // next() does it itself, a driver of many solves before the first next()
+    // so that one solve's host part overlaps the others' device part.
+    int orthogonalise()
+    {
+        if (state != kArnoldi || orthogonal)
+            return T2_OK;
+        T2_HIP(t2::launch_arnoldi(V, n, int(j + 1), V + n * (j + 1), n,
+                                  s->d_red, s->d_scal, s->stream));
+        orthogonal = true;
         return T2_OK;
     }
 
@@ -1355,24 +1368,13 @@ struct Gmres {
                 *need = true;
                 return T2_OK;
             case kArnoldi: {
-                double *w = V + n * (j + 1);
-                for (int pass = 0; pass < 2; pass++) {
-                    T2_HIP(t2::launch_multi_dot(V, n, int(j + 1), w, n,
-                                                s->d_red, s->d_scal,
-                                                s->stream));
-                    T2_HIP(t2::launch_multi_axpy(V, n, int(j + 1), s->d_scal,
-                                                 w, n, s->stream));
-                    T2_TRY(fetch(s, pass ? h2.data() : h.data(), s->d_scal,
-                                 j + 1));
-                }
+                T2_TRY(orthogonalise());
+                orthogonal = false;
+                T2_TRY(fetch(s, h.data(), s->d_scal, t2::kArnoldiScalars));
+                const double *h2 = h.data() + t2::kMaxArnoldi;
                 for (int64_t i = 0; i <= j; i++)
                     H[i * m + j] = h[i] + h2[i];
-                double ww = 0.0;
-                T2_TRY(dot(s, w, w, n, &ww));
-                const double hn = std::sqrt(ww);
-                H[(j + 1) * m + j] = hn;
-                if (hn != 0.0)
-                    T2_HIP(t2::launch_scale(w, 1.0 / hn, n, s->stream));
+                H[(j + 1) * m + j] = std::sqrt(h2[t2::kMaxArnoldi]);
                 for (int64_t i = 0; i < j; i++) {
                     const double t =
                         cs[i] * H[i * m + j] + sn[i] * H[(i + 1) * m + j];
@@ -3267,6 +3269,7 @@ static int batch_gmres(t2_batch *b, std::vector<Gmres> &gm,
             T2_TRY(psi_to_phi(m, gm[i].req_out));
             T2_HIP(t2::launch_axpby(1.0, gm[i].req_in, -1.0, gm[i].req_out,
                                     m->n_phi(), m->stream));
+            T2_TRY(gm[i].orthogonalise());
         }
     }
 }

@@ -314,6 +314,15 @@ hipError_t launch_l1_change(const double *x, const double *y, int64_t n,
 hipError_t launch_multi_dot(const double *V, int64_t ldv, int m,
                             const double *w, int64_t n, double *partial,
                             double *out, hipStream_t stream);
+// An Arnoldi step's orthogonalisation (classical Gram-Schmidt, twice) of w
+// against V[0 .. m): h[0 .. m) and h[kMaxArnoldi ..] the two passes'
+// coefficients, h[2 kMaxArnoldi] the squared norm of what is left, by which w
+// is normalised.  Everything stays on the stream; the caller reads h once.
+constexpr int kMaxArnoldi = 64;
+constexpr int kArnoldiScalars = 2 * kMaxArnoldi + 1;
+hipError_t launch_arnoldi(const double *V, int64_t ldv, int m, double *w,
+                          int64_t n, double *partial, double *h,
+                          hipStream_t stream);
 // w -= sum_j h[j] V[j]  (h on the device)
 hipError_t launch_multi_axpy(const double *V, int64_t ldv, int m,
                              const double *h, double *w, int64_t n,
