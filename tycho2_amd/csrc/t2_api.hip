@@ -699,16 +699,32 @@ int total_source(t2_sweeper *s, const double *q, const double *phi)
     return T2_OK;
 }
 
-int psi_to_phi(t2_sweeper *s, double *phi)
+// phi = D psi, or phi = minus_from - D psi
+int psi_to_phi(t2_sweeper *s, double *phi, const double *minus_from = nullptr)
 {
     if (s->precision == T2_FP64)
         T2_HIP(t2::launch_psi_to_phi<double>(
             static_cast<const double *>(s->d_psi), s->d_wt, s->na,
-            s->n_phi(), phi, s->stream));
+            s->n_phi(), phi, s->stream, minus_from));
     else
         T2_HIP(t2::launch_psi_to_phi<float>(
             static_cast<const float *>(s->d_psi), s->d_wt, s->na, s->n_phi(),
-            phi, s->stream));
+            phi, s->stream, minus_from));
+    return T2_OK;
+}
+
+// phi = D psi and sums = {sum |phi - old|, sum |phi|} (device)
+int psi_to_phi_l1(t2_sweeper *s, double *phi, const double *old,
+                  double *partial, double *sums)
+{
+    if (s->precision == T2_FP64)
+        T2_HIP(t2::launch_psi_to_phi_l1<double>(
+            static_cast<const double *>(s->d_psi), s->d_wt, s->na,
+            s->n_phi(), phi, old, partial, sums, s->stream));
+    else
+        T2_HIP(t2::launch_psi_to_phi_l1<float>(
+            static_cast<const float *>(s->d_psi), s->d_wt, s->na, s->n_phi(),
+            phi, old, partial, sums, s->stream));
     return T2_OK;
 }
 
@@ -1226,9 +1242,7 @@ int transport_apply(t2_sweeper *s, const double *v, double *y)
 {
     T2_TRY(total_source(s, nullptr, v));
     T2_TRY(run_sweep(s, nullptr));
-    T2_TRY(psi_to_phi(s, y));
-    T2_HIP(t2::launch_axpby(1.0, v, -1.0, y, s->n_phi(), s->stream));
-    return T2_OK;
+    return psi_to_phi(s, y, v);
 }
 
 // Restarted GMRES(m) from x = 0: classical Gram-Schmidt applied twice and
@@ -1828,9 +1842,10 @@ static int solve_si_body(t2_sweeper *s, int64_t iter_max, double err_max,
     int64_t it = 0;
     double err = 1.0;
     while (it < iter_max && err > err_max) {
-        T2_TRY(t2_sweep_step(s));
-        T2_HIP(t2::launch_l1_change(s->d_phi, s->d_phi_old, s->n_phi(),
-                                    partial, sums_dev, s->stream));
+        T2_TRY(total_source(s, s->d_qiso, s->d_phi));
+        T2_TRY(run_sweep(s, s->d_qang));
+        std::swap(s->d_phi, s->d_phi_old);
+        T2_TRY(psi_to_phi_l1(s, s->d_phi, s->d_phi_old, partial, sums_dev));
         double sums[2];
         T2_TRY(fetch(s, sums, sums_dev, 2));
         err = sums[0] / sums[1];
@@ -3266,9 +3281,7 @@ static int batch_gmres(t2_batch *b, std::vector<Gmres> &gm,
             if (!act[i])
                 continue;
             t2_sweeper *m = b->members[i];
-            T2_TRY(psi_to_phi(m, gm[i].req_out));
-            T2_HIP(t2::launch_axpby(1.0, gm[i].req_in, -1.0, gm[i].req_out,
-                                    m->n_phi(), m->stream));
+            T2_TRY(psi_to_phi(m, gm[i].req_out, gm[i].req_in));
             T2_TRY(gm[i].orthogonalise());
         }
     }
@@ -3527,9 +3540,8 @@ int t2_batch_solve_source_iteration(t2_batch *b, int64_t iter_max,
                 continue;
             t2_sweeper *m = b->members[i];
             std::swap(m->d_phi, m->d_phi_old);
-            T2_TRY(psi_to_phi(m, m->d_phi));
-            T2_HIP(t2::launch_l1_change(m->d_phi, m->d_phi_old, m->n_phi(),
-                                        m->d_red, m->d_scal, m->stream));
+            T2_TRY(psi_to_phi_l1(m, m->d_phi, m->d_phi_old, m->d_red,
+                                 m->d_scal));
             double sums[2];
             T2_TRY(fetch(m, sums, m->d_scal, 2));
             err[i] = sums[0] / sums[1];

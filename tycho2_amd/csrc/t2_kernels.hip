@@ -1565,19 +1565,44 @@ __global__ void lag_gather_kernel(const int64_t *lag_key,
     lag_buf[i] = v;
 }
 
+__device__ __forceinline__ double block_sum(double v, double *lds)
+{
+    for (int off = 32; off > 0; off >>= 1)
+        v += __shfl_down(v, off, 64);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0)
+        lds[wave] = v;
+    __syncthreads();
+    double s = 0.0;
+    if (threadIdx.x == 0)
+        for (int i = 0; i < int(blockDim.x >> 6); i++)
+            s += lds[i];
+    __syncthreads();
+    return s;  // valid in thread 0
+}
+
 // ---------------------------------------------------------------- moments
 template <typename T>
 struct alignas(16) Vec16 {
     T v[16 / sizeof(T)];
 };
 
-template <typename T>
+// phi = sum_a w_a psi_a; MINUS: phi = x - sum_a w_a psi_a (the Krylov
+// operator); L1: the partial sums of |phi - x| and |phi| as well (the change
+// of a source-iteration step).
+enum MomentMode { kMoment = 0, kMomentMinus = 1, kMomentL1 = 2 };
+
+template <typename T, int MODE>
 __global__ void psi_to_phi_kernel(const T *__restrict__ psi,
                                   const double *__restrict__ wt, int64_t na,
-                                  int64_t n_phi, double *__restrict__ phi)
+                                  int64_t n_phi, double *__restrict__ phi,
+                                  const double *__restrict__ x,
+                                  double *__restrict__ partial)
 {
 #pragma clang fp contract(off)
     constexpr int V = 16 / sizeof(T);
+    __shared__ double lds[16];
+    double s0 = 0.0, s1 = 0.0;
     const int64_t nv = n_phi / V;
     const Vec16<T> *src = reinterpret_cast<const Vec16<T> *>(psi);
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < nv;
@@ -1590,15 +1615,30 @@ __global__ void psi_to_phi_kernel(const T *__restrict__ psi,
         // planes' loads are in flight at once
 #pragma unroll 8
         for (int64_t a = 0; a < na; a++) {
-            const Vec16<T> x = src[size_t(a) * nv + i];
+            const Vec16<T> y = src[size_t(a) * nv + i];
             const double w = wt[a];
 #pragma unroll
             for (int e = 0; e < V; e++)
-                acc[e] += double(x.v[e]) * w;
+                acc[e] += double(y.v[e]) * w;
         }
 #pragma unroll
-        for (int e = 0; e < V; e++)
+        for (int e = 0; e < V; e++) {
+            if constexpr (MODE == kMomentMinus)
+                acc[e] = x[i * V + e] - acc[e];
             phi[i * V + e] = acc[e];
+            if constexpr (MODE == kMomentL1) {
+                s0 += fabs(acc[e] - x[i * V + e]);
+                s1 += fabs(acc[e]);
+            }
+        }
+    }
+    if constexpr (MODE == kMomentL1) {
+        s0 = block_sum(s0, lds);
+        s1 = block_sum(s1, lds);
+        if (threadIdx.x == 0) {
+            partial[blockIdx.x] = s0;
+            partial[gridDim.x + blockIdx.x] = s1;
+        }
     }
 }
 
@@ -1656,22 +1696,6 @@ __global__ void ac_to_ca_kernel(const T *__restrict__ in,
 }
 
 // ---------------------------------------------------------------- reductions
-__device__ __forceinline__ double block_sum(double v, double *lds)
-{
-    for (int off = 32; off > 0; off >>= 1)
-        v += __shfl_down(v, off, 64);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0)
-        lds[wave] = v;
-    __syncthreads();
-    double s = 0.0;
-    if (threadIdx.x == 0)
-        for (int i = 0; i < int(blockDim.x >> 6); i++)
-            s += lds[i];
-    __syncthreads();
-    return s;  // valid in thread 0
-}
-
 __global__ void l1_change_kernel(const double *__restrict__ x,
                                  const double *__restrict__ y, int64_t n,
                                  double *partial)
@@ -2205,11 +2229,41 @@ hipError_t launch_lag_gather(const int64_t *lag_key, const int32_t *lag_up,
 
 template <typename T>
 hipError_t launch_psi_to_phi(const T *psi, const double *wt, int64_t na,
-                             int64_t n_phi, double *phi, hipStream_t stream)
+                             int64_t n_phi, double *phi, hipStream_t stream,
+                             const double *minus_from)
 {
     const int64_t nv = n_phi / (16 / sizeof(T));
-    hipLaunchKernelGGL((psi_to_phi_kernel<T>), dim3(stream_grid(nv)),
-                       dim3(256), 0, stream, psi, wt, na, n_phi, phi);
+    if (minus_from)
+        hipLaunchKernelGGL((psi_to_phi_kernel<T, kMomentMinus>),
+                           dim3(stream_grid(nv)), dim3(256), 0, stream, psi,
+                           wt, na, n_phi, phi, minus_from, nullptr);
+    else
+        hipLaunchKernelGGL((psi_to_phi_kernel<T, kMoment>),
+                           dim3(stream_grid(nv)), dim3(256), 0, stream, psi,
+                           wt, na, n_phi, phi, nullptr, nullptr);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_psi_to_phi_l1(const T *psi, const double *wt, int64_t na,
+                                int64_t n_phi, double *phi,
+                                const double *old, double *partial,
+                                double *out, hipStream_t stream)
+{
+    const int64_t nv = n_phi / (16 / sizeof(T));
+    const int64_t grid = (nv + kRedThreads - 1) / kRedThreads;
+    if (grid > kRedBlocks) {   // more blocks than partial sums
+        const hipError_t e =
+            launch_psi_to_phi<T>(psi, wt, na, n_phi, phi, stream);
+        return e != hipSuccess
+                   ? e
+                   : launch_l1_change(phi, old, n_phi, partial, out, stream);
+    }
+    hipLaunchKernelGGL((psi_to_phi_kernel<T, kMomentL1>),
+                       dim3(unsigned(grid)), dim3(kRedThreads), 0, stream,
+                       psi, wt, na, n_phi, phi, old, partial);
+    hipLaunchKernelGGL(finish_sums_kernel, dim3(2), dim3(kRedThreads), 0,
+                       stream, partial, int(grid), out);
     return hipGetLastError();
 }
 
@@ -2386,7 +2440,10 @@ hipError_t launch_fill(double *x, double v, int64_t n, hipStream_t stream)
                                              T *, hipStream_t);               \
     template hipError_t launch_psi_to_phi<T>(const T *, const double *,       \
                                              int64_t, int64_t, double *,      \
-                                             hipStream_t);                    \
+                                             hipStream_t, const double *);    \
+    template hipError_t launch_psi_to_phi_l1<T>(                              \
+        const T *, const double *, int64_t, int64_t, double *,                \
+        const double *, double *, double *, hipStream_t);                     \
     template hipError_t launch_total_source<T>(const double *,                \
                                                const double *,                \
                                                const double *, int64_t, int,  \

@@ -281,10 +281,20 @@ hipError_t launch_lag_gather(const int64_t *lag_key, const int32_t *lag_up,
                              const uint32_t *nbr, const T *psi, T *lag_buf,
                              hipStream_t stream);
 
-// phi[c][v][g] = sum_a w_a psi[a][c][v][g]  (FP64 accumulation)
+// phi[c][v][g] = sum_a w_a psi[a][c][v][g]  (FP64 accumulation), or, with
+// minus_from, minus_from[c][v][g] less that sum (the Krylov operator's last
+// step in the same pass)
 template <typename T>
 hipError_t launch_psi_to_phi(const T *psi, const double *wt, int64_t na,
-                             int64_t n_phi, double *phi, hipStream_t stream);
+                             int64_t n_phi, double *phi, hipStream_t stream,
+                             const double *minus_from = nullptr);
+// phi as above and launch_l1_change(phi, old), in one pass over phi where
+// its blocks' partial sums fit `partial`
+template <typename T>
+hipError_t launch_psi_to_phi_l1(const T *psi, const double *wt, int64_t na,
+                                int64_t n_phi, double *phi,
+                                const double *old, double *partial,
+                                double *out, hipStream_t stream);
 
 // out[c][v][g] = (q ? q[c][v][g] : 0) + sigma_s[c][g] / (4 pi) * phi[c][v][g]
 template <typename T>
