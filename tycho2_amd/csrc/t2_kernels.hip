@@ -774,6 +774,133 @@ __device__ __forceinline__ void buffer_geo(Rsrc r, uint32_t off,
     g = __builtin_bit_cast(ItemGeo<float>, x);
 }
 
+// x of the lane at quad position (lane ^ X), X = 1 or 2.
+template <int X>
+__device__ __forceinline__ uint32_t quad_swap(uint32_t x)
+{
+    return uint32_t(__builtin_amdgcn_mov_dpp(
+        int(x), X == 1 ? 0xB1 : 0x4E, 0xF, 0xF, true));
+}
+template <int X>
+__device__ __forceinline__ float quad_swap(float x)
+{
+    return __builtin_bit_cast(
+        float, quad_swap<X>(__builtin_bit_cast(uint32_t, x)));
+}
+template <int X>
+__device__ __forceinline__ double quad_swap(double x)
+{
+    struct W {
+        uint32_t lo, hi;
+    } w = __builtin_bit_cast(W, x);
+    w.lo = quad_swap<X>(w.lo);
+    w.hi = quad_swap<X>(w.hi);
+    return __builtin_bit_cast(double, w);
+}
+
+// Between one group's values of the four vertices and pieces of N groups of
+// 4 / N vertices, over N neighbouring lanes: with s the lane's place among
+// them, x[v] = (vertex v, group s) <-> x[N h + j] = (vertex N h + s, group
+// j).  Its own inverse; all lanes take part.
+template <int N, typename X>
+__device__ __forceinline__ void regroup(uint32_t lane, X x[4])
+{
+    if constexpr (N > 1) {
+        const bool odd = lane & 1u;
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+            const X other = quad_swap<1>(odd ? x[i] : x[i + 1]);
+            if (odd)
+                x[i] = other;
+            else
+                x[i + 1] = other;
+        }
+    }
+    if constexpr (N > 2) {
+        const bool odd = lane & 2u;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const X other = quad_swap<2>(odd ? x[i] : x[i + 2]);
+            if (odd)
+                x[i] = other;
+            else
+                x[i + 2] = other;
+        }
+    }
+}
+
+// The groups that one access moves, of GC neighbouring ones of type X.
+template <typename X, int GC>
+constexpr int piece_groups()
+{
+    constexpr int most = 16 / int(sizeof(X));
+    return GC < most ? GC : most;
+}
+__device__ __forceinline__ void buffer_piece(Rsrc r, uint32_t off, double *x,
+                                             std::integral_constant<int, 2>)
+{
+    struct X {
+        double v[2];
+    } y = __builtin_bit_cast(
+        X, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+    x[0] = y.v[0];
+    x[1] = y.v[1];
+}
+__device__ __forceinline__ void buffer_piece(Rsrc r, uint32_t off, float *x,
+                                             std::integral_constant<int, 4>)
+{
+    buffer_row(r, off, x);
+}
+__device__ __forceinline__ void buffer_piece(Rsrc r, uint32_t off, float *x,
+                                             std::integral_constant<int, 2>)
+{
+    struct X {
+        float v[2];
+    } y = __builtin_bit_cast(
+        X, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    x[0] = y.v[0];
+    x[1] = y.v[1];
+}
+template <typename X>
+__device__ __forceinline__ void buffer_piece(Rsrc r, uint32_t off, X *x,
+                                             std::integral_constant<int, 1>)
+{
+    buffer_value(r, off, *x);
+}
+__device__ __forceinline__ void
+buffer_store_piece(Rsrc r, uint32_t off, const double *x,
+                   std::integral_constant<int, 2>)
+{
+    struct X {
+        double v[2];
+    } y = {{x[0], x[1]}};
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(Word4, y), r,
+                                           off, 0, 0);
+}
+__device__ __forceinline__ void
+buffer_store_piece(Rsrc r, uint32_t off, const float *x,
+                   std::integral_constant<int, 4>)
+{
+    buffer_store_row(r, off, x);
+}
+__device__ __forceinline__ void
+buffer_store_piece(Rsrc r, uint32_t off, const float *x,
+                   std::integral_constant<int, 2>)
+{
+    struct X {
+        float v[2];
+    } y = {{x[0], x[1]}};
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(Word2, y), r,
+                                          off, 0, 0);
+}
+template <typename X>
+__device__ __forceinline__ void
+buffer_store_piece(Rsrc r, uint32_t off, const X *x,
+                   std::integral_constant<int, 1>)
+{
+    buffer_store(r, off, *x);
+}
+
 // A block sweeps one angle for GC groups; the values that later levels read
 // stay in the block's LDS (slot form of the records), so that a level hands
 // on to the next without a global round trip.
@@ -791,10 +918,26 @@ __device__ __forceinline__ void buffer_geo(Rsrc r, uint32_t off,
 // The wavefront's LDS operations are performed in order, so a round's values
 // are in LDS before its count is.
 //
+// What a round costs is its accesses, not its bytes or its 430 instructions:
+// a wavefront's 64 values of one vertex lie in 64 / GC cache lines.  So
+// neighbouring lanes trade values (regroup) until each holds 16 bytes, and two
+// or four vertices of a cell leave in one access; and the next round's loads
+// go before the stores, without a branch between them, so that waiting for
+// them does not wait for the stores.  A sweep of 34,992 cells x 128 angles x 4
+// groups FP64: 533 -> 409 us, 2.2 TB/s of its 0.92 GB (252 us without stores,
+// 342 without loads, no less without the waits between levels);
+// 48,000 x 288 x 8 FP32: 1860 -> 1300 us; 24,576 x 32 x 16 FP64, whose rows
+// are lines: 419 -> 403.  Small problems are bound by the levels: 0.54 us each
+// (6,000 x 32 x 4 FP64 in 25 us; step launches 3.6 us a level).
+//
 // ANG: angle-dependent source, 0 none, 1 FP64 (src_ang), 2 T (src_ang_t).
 // ROW: one group in all, so that a cell's four values are contiguous and move
 // in one access.
-template <typename T, int GC, int ANG, bool ROW>
+// PIECES: loads of the sources in 16 bytes too (rows of 16 to 32 bytes gain 3
+// to 9%, longer ones nothing).  Not where the registers would spill: in the
+// kernel of several problems (six problems' GMRES 23.5 instead of 21.3 ms) and
+// with two FP64 sources.
+template <typename T, int GC, int ANG, bool ROW, bool PIECES>
 __device__ __forceinline__ void sweep_angle(const SweepArgs<T> &p,
                                             const AngleSweep &t, int task,
                                             char *lds_raw)
@@ -843,7 +986,8 @@ __device__ __forceinline__ void sweep_angle(const SweepArgs<T> &p,
     __syncthreads();
 
     const int n_rounds = t.round_off[angle + 1] - t.round_off[angle];
-    const AngleRound *const rounds = t.rounds + t.round_off[angle];
+    const Rsrc rounds = buffer_of(t.rounds + t.round_off[angle],
+                                  n_rounds * uint32_t(sizeof(AngleRound)));
     const int n_waves = int(blockDim.x / 64);
     int k = __builtin_amdgcn_readfirstlane(int(threadIdx.x / 64));
     struct Record {
@@ -854,13 +998,25 @@ __device__ __forceinline__ void sweep_angle(const SweepArgs<T> &p,
         T sig, q[4];
         std::conditional_t<ANG == 1, double, T> qa[4];
     };
+    // N groups of a vertex move in one access, from the lane that holds them
+    // after regroup(): of vertices v ... v + N - 1 that of the lane's place
+    constexpr int kN = ROW ? 1 : piece_groups<T, GC>();
+    using Pieces = std::integral_constant<int, kN>;
+    constexpr bool kLoadPieces = PIECES && !(ANG == 1 && sizeof(T) == 8);
+    constexpr int kL = kLoadPieces ? kN : 1;   // ... of a load
+    using Loads = std::integral_constant<int, kL>;
+    const int cg_log = __builtin_ctz(CG);   // G is a power of two
+    auto element = [&](auto n, uint32_t cell, int v) {
+        constexpr uint32_t N = decltype(n)::value;
+        return (cell << cg_log) + ((v + lane % N) * G + g - lane % N);
+    };
     // a round's entry, issued now and made scalar where it is first used (the
     // buffer descriptors below have to be)
+    // (nothing past the last)
     auto round_at = [&](int i) {
-        AngleRound r{0, 0, 0};
-        if (i < n_rounds)
-            r = rounds[i];
-        return r;
+        const auto w = __builtin_amdgcn_raw_buffer_load_b96(
+            rounds, i * uint32_t(sizeof(AngleRound)), 0, 0);
+        return AngleRound{w[0], w[1], w[2]};
     };
     auto uniform = [](const AngleRound &r) {
         return AngleRound{
@@ -880,35 +1036,54 @@ __device__ __forceinline__ void sweep_angle(const SweepArgs<T> &p,
     };
     auto load_inputs = [&](const AngleRound &r, const Record &rec,
                            Inputs &in) {
+        // lanes past the round's items have cell 0 (their record is outside)
+        // and read its values in vain: no branch behind the first of these
+        // loads, so that the wait for them counts exactly the accesses issued
+        // after them
+        const uint32_t cell = rec.a[0];
+        if (by_item)
+            buffer_value(sigma, (cell * G + g) * uint32_t(sizeof(T)), in.sig);
         const Rsrc b = buffer_of(p.geo + r.item,
                                  r.count * uint32_t(sizeof(ItemGeo<T>)));
         buffer_geo(b, li * uint32_t(sizeof(ItemGeo<T>)), in.geo);
-        const bool mine = li < r.count;
-        const uint32_t cell = rec.a[0];
-        if (by_item)
-            buffer_value(sigma,
-                         mine ? (cell * G + g) * uint32_t(sizeof(T))
-                              : kOutside,
-                         in.sig);
         if constexpr (ROW) {
-            buffer_row(src, mine ? cell * 4 * uint32_t(sizeof(T)) : kOutside,
-                       in.q);
+            buffer_row(src, cell * 4 * uint32_t(sizeof(T)), in.q);
             if constexpr (ANG != 0)
-                buffer_row(src_a,
-                           mine ? cell * 4 * uint32_t(sizeof(in.qa[0]))
-                                : kOutside,
+                buffer_row(src_a, cell * 4 * uint32_t(sizeof(in.qa[0])),
                            in.qa);
             return;
         }
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const uint32_t e = cell * CG + g + v * G;
-            buffer_value(src, mine ? e * uint32_t(sizeof(T)) : kOutside,
-                         in.q[v]);
-            if constexpr (ANG != 0)
-                buffer_value(src_a,
-                             mine ? e * uint32_t(sizeof(in.qa[0])) : kOutside,
-                             in.qa[v]);
+        for (int v = 0; v < 4; v += kL)
+            buffer_piece(src,
+                         element(Loads(), cell, v) * uint32_t(sizeof(T)),
+                         &in.q[v], Loads());
+        if constexpr (ANG != 0) {
+            using A = std::remove_reference_t<decltype(in.qa[0])>;
+            using P = std::integral_constant<
+                int, kLoadPieces ? piece_groups<A, GC>() : 1>;
+#pragma unroll
+            for (int v = 0; v < 4; v += P::value)
+                buffer_piece(src_a,
+                             element(P(), cell, v) * uint32_t(sizeof(A)),
+                             &in.qa[v], P());
+        }
+    };
+
+    // plain stores: the other chunks' blocks complete the cache lines
+    auto store_psi = [&](uint32_t cell, bool mine, const T x[4]) {
+        if constexpr (ROW) {
+            const uint32_t dst = cell * 4 * uint32_t(sizeof(T));
+            buffer_store_row(psi_a, mine ? dst : kOutside, x);
+            return;
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v += kN) {
+            uint32_t dst = element(Pieces(), cell, v) * uint32_t(sizeof(T));
+            asm("" : "+v"(dst));   // select, not branch
+            dst = mine ? dst : kOutside;
+            asm volatile("" : "+v"(dst));   // not merged with another store
+            buffer_store_piece(psi_a, dst, &x[v], Pieces());
         }
     };
 
@@ -919,15 +1094,31 @@ __device__ __forceinline__ void sweep_angle(const SweepArgs<T> &p,
     constexpr bool kEarly = sizeof(T) == 4;
     AngleRound r0 = uniform(round_at(k));
     AngleRound r1 = uniform(round_at(k + n_waves));
-    AngleRound r2 = round_at(k + 2 * n_waves);
-    Record rec0 = load_record(r0), rec1 = load_record(r1);
+    Record rec0 = load_record(r0), rec1;
+    AngleRound r2;
     Inputs in;
-    load_inputs(r0, rec0, in);
+    if constexpr (kEarly)
+        load_inputs(r0, rec0, in);
+    rec1 = load_record(r1);
+    r2 = round_at(k + 2 * n_waves);
+    if constexpr (!kEarly)
+        load_inputs(r0, rec0, in);
+    // as many accesses behind these loads as the loop has, so that its wait
+    // for them lets as many stores be outstanding (these store nothing)
+    const T none[4] = {};
+    store_psi(0, false, none);
     for (; k < n_rounds; k += n_waves) {
         // ahead of the earlier levels: this round's factors and LDS
         // addresses, the next one's inputs, the record of the one after it,
         // the entry of the third
         T a12[4], q[4];
+        if constexpr (!ROW) {
+            regroup<kL>(lane, in.q);
+            if constexpr (ANG != 0)
+                regroup<kLoadPieces ? piece_groups<std::remove_reference_t<
+                                          decltype(in.qa[0])>, GC>()
+                                    : 1>(lane, in.qa);
+        }
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             a12[i] = in.geo.a12[i];
@@ -949,7 +1140,7 @@ __device__ __forceinline__ void sweep_angle(const SweepArgs<T> &p,
         }
         const bool mine = li < r0.count;
         const uint32_t own = mine ? rec0.a[1] & 0xFFFFu : uint32_t(kNoValue);
-        const uint32_t dst = (rec0.a[0] * CG + g) * uint32_t(sizeof(T));
+        const uint32_t cell = rec0.a[0];
         const int need = int(r0.need);
         // faces that any lane of the wavefront reads
         bool reads[4];
@@ -1007,19 +1198,13 @@ __device__ __forceinline__ void sweep_angle(const SweepArgs<T> &p,
             __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
         __builtin_amdgcn_s_setprio(0);
-        // plain stores: the other chunks' blocks complete the cache lines
-        if constexpr (ROW) {
-            buffer_store_row(psi_a, mine ? dst : kOutside, f.b);
-        } else {
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                buffer_store(psi_a,
-                             mine ? dst + v * G * uint32_t(sizeof(T))
-                                  : kOutside,
-                             f.b[v]);
-        }
+        // loads before the stores: waiting for them later does not wait for
+        // the stores then
         if constexpr (!kEarly)
             load_inputs(r0, rec0, in);
+        if constexpr (!ROW)
+            regroup<kN>(lane, f.b);
+        store_psi(cell, mine, f.b);
     }
 }
 
@@ -1028,7 +1213,7 @@ __global__ void __launch_bounds__(kMaxAngleBlock)
 angle_sweep_kernel(const SweepArgs<T> p, const AngleSweep t)
 {
     extern __shared__ char lds_raw[];
-    sweep_angle<T, GC, ANG, ROW>(p, t, int(blockIdx.x), lds_raw);
+    sweep_angle<T, GC, ANG, ROW, true>(p, t, int(blockIdx.x), lds_raw);
 }
 
 // Several problems in one launch: each run of blocks sweeps one problem (its
@@ -1036,7 +1221,7 @@ angle_sweep_kernel(const SweepArgs<T> p, const AngleSweep t)
 // Merged step launches gave a small member's levels a share of one launch,
 // but every level of the deepest member its 4 us; here each block runs at its
 // own pace.  Six problems of 2,058 to 24,576 cells, 32 to 288 angles and 1 to
-// 32 groups, FP64 GMRES in lock step: 82.1 -> 31.4 ms a solve.  Blocks of 512
+// 32 groups, FP64 GMRES in lock step: 82.1 -> 21.3 ms a solve.  Blocks of 512
 // threads, two a CU within 128 registers.
 template <typename T, int ANG>
 __global__ void __launch_bounds__(kBatchAngleBlock, 4)
@@ -1065,13 +1250,13 @@ angle_batch_kernel(const AngleProblem<T> *problems, const int2 *runs,
     switch (ap.t.groups / ap.t.chunks) {
     case 1:
         if (ap.t.groups == 1)
-            sweep_angle<T, 1, ANG, true>(ap.a, ap.t, task, lds_raw);
+            sweep_angle<T, 1, ANG, true, false>(ap.a, ap.t, task, lds_raw);
         else
-            sweep_angle<T, 1, ANG, false>(ap.a, ap.t, task, lds_raw);
+            sweep_angle<T, 1, ANG, false, false>(ap.a, ap.t, task, lds_raw);
         break;
-    case 2: sweep_angle<T, 2, ANG, false>(ap.a, ap.t, task, lds_raw); break;
-    case 4: sweep_angle<T, 4, ANG, false>(ap.a, ap.t, task, lds_raw); break;
-    case 8: sweep_angle<T, 8, ANG, false>(ap.a, ap.t, task, lds_raw); break;
+    case 2: sweep_angle<T, 2, ANG, false, false>(ap.a, ap.t, task, lds_raw); break;
+    case 4: sweep_angle<T, 4, ANG, false, false>(ap.a, ap.t, task, lds_raw); break;
+    case 8: sweep_angle<T, 8, ANG, false, false>(ap.a, ap.t, task, lds_raw); break;
     default: break;
     }
 }
