@@ -110,20 +110,6 @@ int build_slots(const HostMesh &m, int64_t na, const double *omega,
                 const Schedule &s, std::vector<uint16_t> &slot,
                 int64_t *n_slots);
 
-// Chain schedule of the level sets' dependency graph: every step holds chains
-// of up to `length` cells of one angle, each cell of a chain reading only
-// cells of earlier steps and earlier cells of its own chain.  A step's work
-// is its chains' first cells, then the second cells of the chains that have
-// one, and so on, chain i at place i of each part (longest chains first).
-constexpr int kMaxChain = 4;
-struct ChainSchedule {
-    int length = 0;
-    std::vector<uint32_t> work;        // [nc * na], cell | angle << cell_bits
-    std::vector<uint32_t> count;       // [steps][length] cells of each part
-};
-int build_chains(const HostMesh &m, int64_t na, const double *omega,
-                 const Schedule &s, int length, ChainSchedule &out);
-
 // Traversal priorities of the reference's graph traverser on one rank
 // (src/Priorities.cc:396-435): intra-angle rule 0 random, 1 b-level,
 // 2 BFDS, 3 DFDS, 4 DFHDS; inter-angle rule 0 interleaved, 1 globally

@@ -639,159 +639,6 @@ void reverse_level_order(const int32_t *level, int64_t nc,
 
 }  // namespace
 
-int build_chains(const HostMesh &m, int64_t na, const double *omega,
-                 const Schedule &s, int length, ChainSchedule &out)
-{
-    const int64_t nc = m.nc;
-    const SweepDag dag(m, na, omega, s.lagged);
-    // one angle: its cells chain by chain in step order, longest chains and
-    // then equal patterns of incoming faces together within a step
-    struct Angle {
-        std::vector<int32_t> cells;
-        std::vector<uint32_t> chains;  // [steps][length]: chains by length
-    };
-    std::vector<Angle> angles(na);
-    for_each_angle(na, [&](int64_t a) {
-        struct Chain {
-            uint32_t key;
-            int32_t cell[kMaxChain];
-        };
-        Angle &an = angles[a];
-        const double *om = omega + 3 * a;
-        std::vector<uint8_t> left(nc), taken(nc, 0), mask(nc, 0);
-        std::vector<int32_t> front, next;
-        std::vector<Chain> step;
-        an.cells.reserve(nc);
-        for (int64_t c = 0; c < nc; c++) {
-            left[c] = uint8_t(dag.in_degree(a, c));
-            if (!left[c]) {
-                front.push_back(int32_t(c));
-                taken[c] = 1;
-            }
-            for (int k = 0; k < 4; k++)
-                if (m.adj[4 * c + k] >= 0 &&
-                    omega_dot_n(om, &m.normal[(4 * c + k) * 3]) < 0)
-                    mask[c] |= uint8_t(1u << k);
-        }
-        while (!front.empty()) {
-            step.clear();
-            for (int32_t head : front) {
-                Chain ch;
-                int n = 0;
-                int64_t down[kMaxChain][4];
-                int n_down[kMaxChain];
-                int32_t cell = head;
-                for (;;) {
-                    ch.cell[n] = cell;
-                    n_down[n] = dag.down(a, cell, down[n]);
-                    n++;
-                    if (n == length)
-                        break;
-                    // the cell that only waits for this chain, and for the
-                    // most of it
-                    int best = 0;
-                    for (int i = 0; i < n; i++)
-                        for (int j = 0; j < n_down[i]; j++) {
-                            const int64_t d = down[i][j];
-                            if (taken[d])
-                                continue;
-                            int own = 0;
-                            for (int q = 0; q < n; q++)
-                                for (int r = 0; r < n_down[q]; r++)
-                                    own += down[q][r] == d;
-                            if (own == left[d] && own > best) {
-                                best = own;
-                                cell = int32_t(d);
-                            }
-                        }
-                    if (!best)
-                        break;
-                    taken[cell] = 1;
-                }
-                ch.key = uint32_t(kMaxChain - n) << 16;
-                for (int i = 0; i < n; i++)
-                    ch.key |= uint32_t(mask[ch.cell[i]]) << (4 * (3 - i));
-                step.push_back(ch);
-            }
-            std::stable_sort(step.begin(), step.end(),
-                             [](const Chain &x, const Chain &y) {
-                                 return x.key < y.key;
-                             });
-            const size_t at = an.chains.size();
-            an.chains.resize(at + length, 0);
-            next.clear();
-            for (const Chain &ch : step) {
-                const int n = kMaxChain - int(ch.key >> 16);
-                an.chains[at + n - 1]++;
-                for (int i = 0; i < n; i++) {
-                    an.cells.push_back(ch.cell[i]);
-                    int64_t down[4];
-                    const int nd = dag.down(a, ch.cell[i], down);
-                    for (int j = 0; j < nd; j++)
-                        if (--left[down[j]] == 0 && !taken[down[j]]) {
-                            taken[down[j]] = 1;
-                            next.push_back(int32_t(down[j]));
-                        }
-                }
-            }
-            front.swap(next);
-        }
-    });
-    size_t steps = 0;
-    for (const Angle &an : angles)
-        steps = std::max(steps, an.chains.size() / length);
-    // chains of a step by length (longest first) and angle
-    out.length = length;
-    out.count.assign(steps * length, 0);
-    std::vector<size_t> base(steps + 1, 0);
-    std::vector<std::vector<uint32_t>> at(na);   // first chain's place
-    {
-        std::vector<uint32_t> place(steps, 0);
-        for (int n = length; n >= 1; n--)
-            for (int64_t a = 0; a < na; a++) {
-                const Angle &an = angles[a];
-                at[a].resize(an.chains.size());
-                for (size_t st = 0; st < an.chains.size() / length; st++) {
-                    const uint32_t k = an.chains[st * length + n - 1];
-                    at[a][st * length + n - 1] = place[st];
-                    place[st] += k;
-                    for (int p = 0; p < n; p++)
-                        out.count[st * length + p] += k;
-                }
-            }
-    }
-    for (size_t st = 0; st < steps; st++) {
-        base[st + 1] = base[st];
-        for (int p = 0; p < length; p++)
-            base[st + 1] += out.count[st * length + p];
-    }
-    if (base[steps] != size_t(na) * nc)
-        return fail(T2_ERR_ARG, "chain schedule: dependency graph left "
-                                "items unscheduled");
-    try {
-        out.work.resize(size_t(na) * nc);
-    } catch (...) {
-        return fail(T2_ERR_NOMEM, "host memory for the chain schedule");
-    }
-    for_each_angle(na, [&](int64_t a) {
-        const Angle &an = angles[a];
-        const int32_t *c = an.cells.data();
-        for (size_t st = 0; st < an.chains.size() / length; st++)
-            for (int n = length; n >= 1; n--) {
-                const uint32_t first = at[a][st * length + n - 1];
-                for (uint32_t i = 0; i < an.chains[st * length + n - 1]; i++) {
-                    size_t part = base[st];
-                    for (int p = 0; p < n; p++) {
-                        out.work[part + first + i] =
-                            uint32_t(*c++) | (uint32_t(a) << s.cell_bits);
-                        part += out.count[st * length + p];
-                    }
-                }
-            }
-    });
-    return T2_OK;
-}
-
 int sweep_priorities(const HostMesh &m, int64_t na, const double *omega,
                      const int32_t *levels,
                      const std::vector<LaggedFace> &lagged, int intra,
