@@ -929,16 +929,24 @@ int angle_groups(const t2_sweeper *s, int64_t slots)
 }
 
 // Whether that form is faster than the step launches: its bytes per solve
-// (records once per gc groups, source and psi) at the 3 TB/s it reaches
-// against 3.6 us per step and the step launches' 13.5 values per solve at
-// 5.2 TB/s, more of them wasted the shorter a vertex row is than 32 bytes.
-// Measured a sweep, angle form / step launches (us):
-//   750 cells,  32 angles, 1 group,  FP64    34 /   179
-//   34,992     128          4        FP64   533 /  1471
-//   48,000     288          8        FP32  1875 /  2778
-//   73,002     128         16        FP32  3136 /  2560 (not taken)
-//   384,000    128          1        FP32  2760 /  5227
-//   196,608    128          4        FP64  4530 /  4450 (not taken)
+// (records once per gc groups, source and psi) at the rate it reaches against
+// 3.6 us per step and the step launches' 13.5 values per solve at 5.2 TB/s,
+// more of them wasted the shorter a vertex row is than 32 bytes.  The rate is
+// 4 TB/s where a row is in at most four parts of two or more groups, 3 TB/s
+// otherwise: more parts or smaller ones keep up with each other only while
+// the handle has the chip to itself.  Measured, angle form / step launches (us), a sweep
+// alone and a Krylov apply among those of three handles:
+//      750 cells,  32 angles, 1 group,  FP64    34 /   179
+//   34,992        128          4        FP64   410 /  1260
+//   48,000        288          8        FP32  1300 /  2778
+//   73,002        128         16        FP32  1708 /  2568    2140 / 2247
+//  131,712        128          8        FP32  1939 /  3176    2316 / 2517
+//  384,000        128          2        FP32  3780 /  6340    4074 / 4932
+//   73,002        128         16        FP64  3684 /  3930    5921 / 3757 *
+//   82,944        128         32        FP32  4385 /  4615    6944 / 4463 *
+//   82,944        288          4        FP64  3474 /  3460    3732 / 3089 *
+//  131,712        128          4        FP64  2309 /  2814    2927 / 2326 *
+// (* not taken).
 bool angle_pays(const t2_sweeper *s, int gc)
 {
     if (gc <= 0)
@@ -948,9 +956,12 @@ bool angle_pays(const t2_sweeper *s, int gc)
                        double(s->precision == T2_FP64
                                   ? sizeof(t2::ItemGeo<double>)
                                   : sizeof(t2::ItemGeo<float>));
+    const int64_t parts = s->ng / gc;
+    const double rate =
+        parts == 1 || (parts <= 4 && gc >= 2) ? 4.0e12 : 3.0e12;
     const double solves = double(s->nc) * double(s->na) * double(s->ng);
     const double waste = std::max(1.0, 32.0 / (w * double(s->ng)));
-    return solves * (rec / gc + 8.0 * w) / 3.0e12 <
+    return solves * (rec / gc + 8.0 * w) / rate <
            3.6e-6 * double(s->sched.n_steps) +
                solves * 13.5 * w * waste / 5.2e12;
 }
