@@ -255,6 +255,107 @@ __global__ void build_items_kernel(const uint32_t *__restrict__ work,
     out_topo[i] = rt;
 }
 
+// x of the lane at quad position (lane ^ X), X = 1 or 2.
+template <int X>
+__device__ __forceinline__ uint32_t quad_swap(uint32_t x)
+{
+    return uint32_t(__builtin_amdgcn_mov_dpp(
+        int(x), X == 1 ? 0xB1 : 0x4E, 0xF, 0xF, true));
+}
+template <int X>
+__device__ __forceinline__ float quad_swap(float x)
+{
+    return __builtin_bit_cast(
+        float, quad_swap<X>(__builtin_bit_cast(uint32_t, x)));
+}
+template <int X>
+__device__ __forceinline__ double quad_swap(double x)
+{
+    struct W {
+        uint32_t lo, hi;
+    } w = __builtin_bit_cast(W, x);
+    w.lo = quad_swap<X>(w.lo);
+    w.hi = quad_swap<X>(w.hi);
+    return __builtin_bit_cast(double, w);
+}
+
+// Between one group's values of the four vertices and pieces of N groups of
+// 4 / N vertices, over N neighbouring lanes: with s the lane's place among
+// them, x[v] = (vertex v, group s) <-> x[N h + j] = (vertex N h + s, group
+// j).  Its own inverse; all lanes take part.
+template <int N, typename X>
+__device__ __forceinline__ void regroup(uint32_t lane, X x[4])
+{
+    if constexpr (N > 1) {
+        const bool odd = lane & 1u;
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+            const X other = quad_swap<1>(odd ? x[i] : x[i + 1]);
+            if (odd)
+                x[i] = other;
+            else
+                x[i + 1] = other;
+        }
+    }
+    if constexpr (N > 2) {
+        const bool odd = lane & 2u;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const X other = quad_swap<2>(odd ? x[i] : x[i + 2]);
+            if (odd)
+                x[i] = other;
+            else
+                x[i + 2] = other;
+        }
+    }
+}
+
+// The groups that one access moves, of GC neighbouring ones of type X.
+template <typename X, int GC>
+constexpr int piece_groups()
+{
+    constexpr int most = 16 / int(sizeof(X));
+    return GC < most ? GC : most;
+}
+// A load or store of N neighbouring values.
+template <int N, typename T>
+struct Piece {
+    typedef T Vec __attribute__((ext_vector_type(N)));
+    static __device__ __forceinline__ void load(const T *from, T *x)
+    {
+        const Vec v = *reinterpret_cast<const Vec *>(from);
+#pragma unroll
+        for (int j = 0; j < N; j++)
+            x[j] = v[j];
+    }
+    template <bool STREAM>
+    static __device__ __forceinline__ void store(const T *x, T *to)
+    {
+        Vec v;
+#pragma unroll
+        for (int j = 0; j < N; j++)
+            v[j] = x[j];
+        if constexpr (STREAM)
+            __builtin_nontemporal_store(v, reinterpret_cast<Vec *>(to));
+        else
+            *reinterpret_cast<Vec *>(to) = v;
+    }
+};
+
+// Groups per access of the step launches: 16 bytes of a vertex row of up to
+// 32 bytes, traded between the lanes (regroup), else a lane's own value.
+// Longer rows fill cache lines as they are and gain nothing (FP32 rows of 64
+// bytes lose 1.5% by the loads).  A sweep of 384,000 cells x 128 angles, lane
+// values / pieces (us): FP32 4 groups 7809 / 6165 (5683 with the upwind cells'
+// values too), 8 groups 7463 / 6506 (upwind too: 6557), FP64 2 groups 6564 /
+// 6135 (6257), 4 groups 6637 / 6239 (6473).
+template <typename T, int G, int GPL, bool COH>
+constexpr int step_piece()
+{
+    return GPL == 1 && !COH && G * int(sizeof(T)) <= 32 ? piece_groups<T, G>()
+                                                        : 1;
+}
+
 // ---------------------------------------------------------------- sweep
 // Cell solve of work item `item` (topology record t) for the groups of lane
 // gl: gl, gl + LPI, ... (LPI = G / GPL lanes per item).  COH: upwind psi is
@@ -271,6 +372,9 @@ __device__ __forceinline__ void solve_item(const SweepArgs<T> &p,
 {
     constexpr int LPI = G / GPL;          // lanes per work item
     constexpr uint32_t CG = 4 * G;        // values per (cell, angle)
+    constexpr int kW = step_piece<T, G, GPL, COH>();
+    // upwind cells too where one access a lane takes all their values
+    constexpr bool kFaceRows = kW == 4 && G == 4;
     // record fields as values (a local copy of the whole record would be
     // placed in scratch memory by the sigma selection below)
     const ItemGeo<T> *gp = p.geo + item;
@@ -308,6 +412,8 @@ __device__ __forceinline__ void solve_item(const SweepArgs<T> &p,
 #pragma unroll
     for (int jg = 0; jg < GPL; jg++) {
         const int g = gl + jg * LPI;
+        // the lane's place in an item's values: vertex g % kW of kW
+        const int at = (g % kW) * G + g - g % kW;
         T sig = ge_sig;
         if (sigma_mode != kSigmaCell)
             sig = sigma[sigma_mode == kSigmaGroup ? uint32_t(g)
@@ -316,9 +422,11 @@ __device__ __forceinline__ void solve_item(const SweepArgs<T> &p,
 
         // source: V/20 (q_i + sum_j q_j)  (Transport.cc:58-72)
         T q[4];
+        const T *q_iso = src_iso + own + at;
 #pragma unroll
-        for (int v = 0; v < 4; v++)
-            q[v] = src_iso[own + v * G + g];
+        for (int v = 0; v < 4; v += kW)
+            Piece<kW, T>::load(q_iso + v * G, &q[v]);
+        regroup<kW>(uint32_t(g), q);
         if (p.src_ang) {
             const double *qa = p.src_ang + size_t(t.angle) * plane + own + g;
 #pragma unroll
@@ -345,7 +453,25 @@ __device__ __forceinline__ void solve_item(const SweepArgs<T> &p,
             if (u == -1)
                 continue;
             T uv[4];
-            if (u >= 0) {
+            if (kFaceRows && u >= 0) {
+                // all lanes of an item take this branch
+                T w[4];
+                Piece<4, T>::load(psi_a + uint32_t(u) * CG + at, w);
+                regroup<kW>(uint32_t(g), w);
+                int slot = 0;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if (j == k) {
+                        uv[j] = T(0);
+                        continue;
+                    }
+                    const uint32_t vtx = t.meta >> (6 * k + 2 * slot);
+                    const T lo = vtx & 1u ? w[1] : w[0];
+                    const T hi = vtx & 1u ? w[3] : w[2];
+                    uv[j] = vtx & 2u ? hi : lo;
+                    slot++;
+                }
+            } else if (u >= 0) {
                 const T *pn = psi_a + uint32_t(u) * CG + g;
                 int slot = 0;
 #pragma unroll
@@ -389,20 +515,17 @@ __device__ __forceinline__ void solve_item(const SweepArgs<T> &p,
         else
             solve_nopivot<T>(m, b);
 
-        T *dst = psi + size_t(t.angle) * plane + own + g;
+        T *dst = psi + size_t(t.angle) * plane + own + at;
         if constexpr (COH) {
 #pragma unroll
             for (int v = 0; v < 4; v++)
                 __hip_atomic_store(dst + v * G, b[v], __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
         } else {
+            regroup<kW>(uint32_t(g), b);
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                if constexpr (STREAM)
-                    __builtin_nontemporal_store(b[v], dst + v * G);
-                else
-                    dst[v * G] = b[v];
-            }
+            for (int v = 0; v < 4; v += kW)
+                Piece<kW, T>::template store<STREAM>(&b[v], dst + v * G);
         }
     }
 }
@@ -774,68 +897,6 @@ __device__ __forceinline__ void buffer_geo(Rsrc r, uint32_t off,
     g = __builtin_bit_cast(ItemGeo<float>, x);
 }
 
-// x of the lane at quad position (lane ^ X), X = 1 or 2.
-template <int X>
-__device__ __forceinline__ uint32_t quad_swap(uint32_t x)
-{
-    return uint32_t(__builtin_amdgcn_mov_dpp(
-        int(x), X == 1 ? 0xB1 : 0x4E, 0xF, 0xF, true));
-}
-template <int X>
-__device__ __forceinline__ float quad_swap(float x)
-{
-    return __builtin_bit_cast(
-        float, quad_swap<X>(__builtin_bit_cast(uint32_t, x)));
-}
-template <int X>
-__device__ __forceinline__ double quad_swap(double x)
-{
-    struct W {
-        uint32_t lo, hi;
-    } w = __builtin_bit_cast(W, x);
-    w.lo = quad_swap<X>(w.lo);
-    w.hi = quad_swap<X>(w.hi);
-    return __builtin_bit_cast(double, w);
-}
-
-// Between one group's values of the four vertices and pieces of N groups of
-// 4 / N vertices, over N neighbouring lanes: with s the lane's place among
-// them, x[v] = (vertex v, group s) <-> x[N h + j] = (vertex N h + s, group
-// j).  Its own inverse; all lanes take part.
-template <int N, typename X>
-__device__ __forceinline__ void regroup(uint32_t lane, X x[4])
-{
-    if constexpr (N > 1) {
-        const bool odd = lane & 1u;
-#pragma unroll
-        for (int i = 0; i < 4; i += 2) {
-            const X other = quad_swap<1>(odd ? x[i] : x[i + 1]);
-            if (odd)
-                x[i] = other;
-            else
-                x[i + 1] = other;
-        }
-    }
-    if constexpr (N > 2) {
-        const bool odd = lane & 2u;
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const X other = quad_swap<2>(odd ? x[i] : x[i + 2]);
-            if (odd)
-                x[i] = other;
-            else
-                x[i + 2] = other;
-        }
-    }
-}
-
-// The groups that one access moves, of GC neighbouring ones of type X.
-template <typename X, int GC>
-constexpr int piece_groups()
-{
-    constexpr int most = 16 / int(sizeof(X));
-    return GC < most ? GC : most;
-}
 __device__ __forceinline__ void buffer_piece(Rsrc r, uint32_t off, double *x,
                                              std::integral_constant<int, 2>)
 {
