@@ -907,12 +907,13 @@ void free_angle_form(t2_sweeper *s)
 // as it has bytes): many small parts drift apart and psi's cache lines leave
 // half written.  Step launches against that form, us a pass with three handles
 // at work: 93,750 cells x 72 angles x 32 groups FP64 in 32 parts of 8 bytes
-// 8,200 / 18,400; 162,000 x 128 x 4 FP32 in 2 parts of 8 bytes 2,797 / 2,288;
-// 93,750 x 32 x 4 FP64 in 4 of 8 bytes 668 / 547; 384,000 x 128 x 2 FP32 in 2
-// of 4 bytes 4,958 / 4,543.  Of those, the most groups that leave
+// 5,430 / 18,700; 162,000 x 128 x 4 FP32 in 2 parts of 8 bytes 2,017 / 1,600;
+// 93,750 x 32 x 4 FP64 in 4 of 8 bytes 664 / 480; 384,000 x 128 x 2 FP32 in 2
+// of 4 bytes 4,267 / 4,064.  Of those, the most groups that leave
 // kMinAngleBlocks blocks, because a block's records are read once per gc
-// groups (6,000 cells x 32 angles x 16 groups in FP64: 114, 121 and 165 us a
-// sweep with 256, 128 and 64 blocks).
+// groups.  256, 128 and 64 blocks, us: 24,576 cells x 32 angles x 16 groups
+// FP64 a sweep alone 335, 398, 843, a pass among three handles 417, 326, 496;
+// 6,000 x 32 x 16 87, 93, 131 and 114, 79, 79.
 constexpr int64_t kMinAngleBlocks = 128;
 
 int angle_groups(const t2_sweeper *s, int64_t slots)
@@ -937,15 +938,15 @@ int angle_groups(const t2_sweeper *s, int64_t slots)
 // the handle has the chip to itself.  Measured, angle form / step launches (us), a sweep
 // alone and a Krylov apply among those of three handles:
 //      750 cells,  32 angles, 1 group,  FP64    34 /   179
-//   34,992        128          4        FP64   410 /  1260
-//   48,000        288          8        FP32  1300 /  2778
+//   34,992        128          4        FP64   411 /  1291     481 /  733
+//   48,000        288          8        FP32  1291 /  2267    1330 / 1772
 //   73,002        128         16        FP32  1708 /  2568    2140 / 2247
-//  131,712        128          8        FP32  1939 /  3176    2316 / 2517
-//  384,000        128          2        FP32  3780 /  6340    4074 / 4932
+//  131,712        128          8        FP32  1932 /  2905    2348 / 2234
+//  384,000        128          2        FP32  3754 /  5785    4064 / 4267
+//  384,000        128          1        FP32  2725 /  5056    1841 / 3613
 //   73,002        128         16        FP64  3684 /  3930    5921 / 3757 *
 //   82,944        128         32        FP32  4385 /  4615    6944 / 4463 *
-//   82,944        288          4        FP64  3474 /  3460    3732 / 3089 *
-//  131,712        128          4        FP64  2309 /  2814    2927 / 2326 *
+//  131,712        128          4        FP64  2318 /  2777    2962 / 2153 *
 // (* not taken).
 bool angle_pays(const t2_sweeper *s, int gc)
 {
@@ -976,12 +977,13 @@ int build_angle_tables(t2_sweeper *s)
         s->gauss != T2_GAUSS_NOPIVOT ||
         s->n_phi() * int64_t(sizeof(double)) >= (int64_t(1) << 32))
         return T2_OK;
-    // at least about half of the widest level is live at once: do not look
-    // for slots that could not fit or would not pay
+    // nearly all of the widest level is live when it ends (its cells on the
+    // outflow boundary are not; on Kuhn cubes the table is twice as long): do
+    // not look for slots that could not fit or would not pay
     uint32_t width = 0;
     for (const auto &sl : sc.slice)
         width = std::max(width, sl.count);
-    if (!angle_pays(s, angle_groups(s, width / 2)))
+    if (!angle_pays(s, angle_groups(s, int64_t(width) * 9 / 10)))
         return T2_OK;
     std::vector<int32_t> lag_off(na + 1, 0);
     for (const auto &l : sc.lagged)

@@ -988,8 +988,9 @@ buffer_store_piece(Rsrc r, uint32_t off, const X *x,
 // groups FP64: 533 -> 409 us, 2.2 TB/s of its 0.92 GB (252 us without stores,
 // 342 without loads, no less without the waits between levels);
 // 48,000 x 288 x 8 FP32: 1860 -> 1300 us; 24,576 x 32 x 16 FP64, whose rows
-// are lines: 419 -> 403.  Small problems are bound by the levels: 0.54 us each
-// (6,000 x 32 x 4 FP64 in 25 us; step launches 3.6 us a level).
+// are lines: 419 -> 403.  Small problems are bound by the levels: 0.5 to
+// 0.6 us each (750 x 32 x 1 FP64 in 24 us, 6,000 x 32 x 4 in 62; step launches
+// take 3.6 us a level).
 //
 // ANG: angle-dependent source, 0 none, 1 FP64 (src_ang), 2 T (src_ang_t).
 // ROW: one group in all, so that a cell's four values are contiguous and move
@@ -1282,7 +1283,7 @@ angle_sweep_kernel(const SweepArgs<T> p, const AngleSweep t)
 // Merged step launches gave a small member's levels a share of one launch,
 // but every level of the deepest member its 4 us; here each block runs at its
 // own pace.  Six problems of 2,058 to 24,576 cells, 32 to 288 angles and 1 to
-// 32 groups, FP64 GMRES in lock step: 82.1 -> 21.3 ms a solve.  Blocks of 512
+// 32 groups, FP64 GMRES in lock step: 82 -> 21 ms a solve.  Blocks of 512
 // threads, two a CU within 128 registers.
 template <typename T, int ANG>
 __global__ void __launch_bounds__(kBatchAngleBlock, 4)
@@ -1833,9 +1834,12 @@ struct alignas(16) Vec16 {
     T v[16 / sizeof(T)];
 };
 
-// phi = sum_a w_a psi_a; MINUS: phi = x - sum_a w_a psi_a (the Krylov
-// operator); L1: the partial sums of |phi - x| and |phi| as well (the change
-// of a source-iteration step).
+// phi = sum_a w_a psi_a; kMomentMinus: phi = x - sum_a w_a psi_a (the Krylov
+// operator); kMomentL1: the partial sums of |phi - x| and |phi| as well (the
+// change of a source-iteration step).  Bound by reading psi, 5 to 5.5 TB/s
+// (34,992 cells x 128 angles x 4 groups FP64 in 115 us); at small sizes by its
+// launch, so what follows it on phi is done here: 21 steps of source iteration
+// on 750 x 32 x 1 FP64 1300 -> 1240 us.
 enum MomentMode { kMoment = 0, kMomentMinus = 1, kMomentL1 = 2 };
 
 template <typename T, int MODE>
@@ -2020,9 +2024,9 @@ __global__ void multi_axpy_kernel(const double *__restrict__ V, int64_t ldv,
 // read of V for both (classical Gram-Schmidt's second pass), the values of
 // an element's vectors in registers (M >= m; 48 and 78 registers for 8 and 16,
 // 24 would spill).  With it an Arnoldi step reads the basis three times
-// instead of four and its host part waits once instead of three times: GMRES
-// of 34,992 cells x 128 angles x 4 groups FP64 9.1 -> 8.5 ms, of six problems
-// in lock step 26.1 -> 22.4 ms.
+// instead of four and its host part waits once instead of three times: 0.6 ms
+// less of GMRES of 34,992 cells x 128 angles x 4 groups FP64 (now 7.1 ms) and
+// 3.7 of six problems' in lock step (now 21).
 template <int M>
 __global__ void __launch_bounds__(kRedThreads)
 axpy_dot_kernel(const double *__restrict__ V, int64_t ldv, int m,
