@@ -86,6 +86,7 @@ struct t2_sweeper {
     double *d_sigt64 = nullptr;      // FP64 copy (FP32 handles: residual)
     uint32_t *d_nbr = nullptr;
     // schedule-dependent
+    int64_t generation = 0;          // counts the schedules built so far
     void *d_item_geo = nullptr;      // ItemGeo<T> in step order
     t2::ItemGeo<double> *d_item_geo64 = nullptr;  // FP32 handles: residual
     t2::ItemTopo *d_item_topo = nullptr;
@@ -1078,6 +1079,7 @@ void free_schedule(t2_sweeper *s)
 {
     const size_t n_items = size_t(s->nc) * s->na;
     const int64_t n_lag = int64_t(s->sched.lagged.size());
+    s->generation++;
     drop_graphs(s);
     free_queue(s);
     free_angle_form(s);
@@ -2378,12 +2380,13 @@ struct t2_batch {
 
 namespace {
 
+// The schedule goes by its generation: a rebuilt one often lies at the old
+// one's addresses.
 std::vector<const void *> member_buffers(const t2_sweeper *m)
 {
-    return {m->d_item_geo, m->d_item_topo, m->d_psi, m->d_src, m->d_lag_buf,
-            m->d_lag_key, m->d_sigt, m->d_qang, m->d_pending, m->d_down,
+    return {m->d_psi, m->d_src, m->d_sigt, m->d_qang, m->d_pending, m->d_down,
             m->d_slot_items, m->d_rounds, m->d_angles,
-            reinterpret_cast<const void *>(intptr_t(m->sched.n_steps))};
+            reinterpret_cast<const void *>(intptr_t(m->generation))};
 }
 
 void batch_snapshot(t2_batch *b)
