@@ -92,6 +92,7 @@ def path_leg(p, precision, steps, warmup, ev, tune, solve, launch="",
         info = s.info()
         out["engine"] = info["engine"]
         out["queue_first_step"] = info["queue_first_step"]
+        out["groups_per_block"] = s.form()   # one launch, 0: step launches
         out["streams"] = (info["angle_batches"]
                           if info["concurrent_batches"] else 1)
         for _ in range(warmup):
@@ -722,6 +723,9 @@ def main() -> int:
             kernel = (f"sweep_step_kernel<{ty},{p.ng},{gpl}> (steps before "
                       f"{r['queue_first_step']}) + queue_sweep_kernel")
             launches = r["queue_first_step"] + 1
+        elif r.get("groups_per_block"):
+            kernel = f"angle_sweep_kernel<{ty},{r['groups_per_block']}>"
+            launches = 1
         else:
             kernel = f"sweep_step_kernel<{ty},{p.ng},{gpl}>"
             launches = r["n_steps"]

@@ -168,9 +168,22 @@ int t2_sweeper_create(t2_sweeper **out, int device,
 int t2_sweeper_destroy(t2_sweeper *s);
 int t2_sweeper_info(const t2_sweeper *s, t2_info *info);
 
-/* Launch shape: cells per block and groups per lane (autotuner knobs);
- * 0 keeps the default. */
+/* Launch shape of the step launches and the ready queue: cells per block and
+ * groups per lane (autotuner knobs); 0 keeps what is set.  A number of cells
+ * per block also sets T2_FORM_STEPS. */
 int t2_set_launch(t2_sweeper *s, int items_per_block, int groups_per_lane);
+
+/* Form of the level engine's sweeps.  T2_FORM_AUTO (default): small and deep
+ * problems in one launch, a block sweeping an angle through its levels, while
+ * the knobs of the step launches (groups and items per lane, angle batches)
+ * are at their defaults; T2_FORM_STEPS: one launch per schedule step whatever
+ * the problem.  Results are bitwise the same. */
+#define T2_FORM_AUTO 0
+#define T2_FORM_STEPS 1
+int t2_set_form(t2_sweeper *s, int form);
+/* Groups a block of the one launch sweeps, 0 where a level-engine sweep of
+ * the handle, as it is set now, makes step launches. */
+int t2_get_form(const t2_sweeper *s, int *groups_per_block);
 
 /* Items per lane of the level engine's step launches (1 or 2; NoPivot cell
  * solver and one group per lane only): with 2 a wavefront solves two sets
@@ -231,10 +244,8 @@ int t2_set_priority(t2_sweeper *s, int intra_angle_p, int inter_angle_p,
 
 /* Sweep engine (GraphTraverser::traverse, src/GraphTraverser.cc:467-759):
  *   T2_ENGINE_LEVELS  one kernel launch per schedule step, the whole sweep
- *                     captured once in a hipGraph and replayed (default); with
- *                     the launch and schedule knobs at their defaults, small
- *                     and deep problems run in one launch instead, a block
- *                     sweeping an angle through its levels;
+ *                     captured once in a hipGraph and replayed, or one launch
+ *                     in all (t2_set_form; default);
  *   T2_ENGINE_QUEUE   one persistent launch: blocks take chunks of items in
  *                     schedule order from a device ticket counter, each item
  *                     waits on its atomic pending-upwind counter, solves, and

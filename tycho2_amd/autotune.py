@@ -5,8 +5,9 @@ stream) over
   * angle batches  -- how many octant-ordered groups of angles are swept one
     after the other (smaller per-step working set, more steps), or side by
     side on parallel streams,
-  * cells per block and groups per lane -- the launch shape of the sweep
-    kernels,
+  * the level engine's form -- one launch with a block per angle, where the
+    handle has it, or step launches, and
+  * their cells per block and groups per lane -- the launch shape,
   * the engine -- per-step launches replayed from a hipGraph, one
     persistent ready-queue launch, or per-step launches with the schedule's
     thin tail on the ready queue (and the queue's chunk size),
@@ -17,7 +18,7 @@ Results do not depend on any of these knobs (bitwise, tested).
 """
 from __future__ import annotations
 
-from .sweeper import ENGINE_HYBRID, ENGINE_LEVELS, ENGINE_QUEUE
+from .sweeper import ENGINE_HYBRID, ENGINE_LEVELS, ENGINE_QUEUE, FORM_AUTO
 from .timing import HipEvents, time_region
 
 BATCHES = (1, 2, 4, 8, 16)
@@ -39,17 +40,32 @@ def tune(s, reps: int = 3, batches=BATCHES, blocks=BLOCKS,
          engines=(ENGINE_LEVELS, ENGINE_QUEUE, ENGINE_HYBRID), log=None,
          priorities=()):
     """Tune handle `s` in place; returns (best, trials) where best is a dict
-    {engine, batches, block, groups_per_lane, ms[, chunk_rounds,
-    priority]} and trials lists every timing; log (a callable) receives one
-    line per trial.  priorities: (intraAngleP, interAngleP, maxCellsPerStep)
-    rules tried on the ready queue after the rest (each rebuilds the
-    schedule on the host)."""
+    {engine, batches, block, groups_per_lane, one_launch, ms[,
+    chunk_rounds, priority]} and trials lists every timing (one_launch: the
+    level engine's form with a block per angle, which has no launch shape);
+    log (a callable) receives one line per trial.  priorities: (intraAngleP,
+    interAngleP, maxCellsPerStep) rules tried on the ready queue after the
+    rest (each rebuilds the schedule on the host)."""
     ev = HipEvents()
     ng = s.ng
     trials = []
     best = None
     s.set_engine(ENGINE_LEVELS)
     s.set_items_per_lane(1)
+    s.set_schedule(1)
+    s.set_concurrent_batches(False)
+    s.set_launch(0, 1)
+    # one launch, to be compared with the best of the rest
+    s.set_form(FORM_AUTO)
+    one = None
+    if s.form():
+        ms = _time_sweep(ev, s, reps)
+        one = dict(engine=ENGINE_LEVELS, batches=1, concurrent=False,
+                   block=256, groups_per_lane=1, items_per_lane=1,
+                   one_launch=True, ms=ms)
+        trials.append(one)
+        if log:
+            log(f"tune {one}")
     # schedule first (it rebuilds the records), with the default launch;
     # several angle batches one after the other or side by side
     for nb in batches:
@@ -61,7 +77,8 @@ def tune(s, reps: int = 3, batches=BATCHES, blocks=BLOCKS,
             s.set_concurrent_batches(conc)
             ms = _time_sweep(ev, s, reps)
             t = dict(engine=ENGINE_LEVELS, batches=nb, concurrent=conc,
-                     block=256, groups_per_lane=1, items_per_lane=1, ms=ms)
+                     block=256, groups_per_lane=1, items_per_lane=1,
+                     one_launch=False, ms=ms)
             trials.append(t)
             if log:
                 log(f"tune {t}")
@@ -80,7 +97,8 @@ def tune(s, reps: int = 3, batches=BATCHES, blocks=BLOCKS,
             ms = _time_sweep(ev, s, reps)
             t = dict(engine=ENGINE_LEVELS, batches=best["batches"],
                      concurrent=best["concurrent"], block=block,
-                     groups_per_lane=gpl, items_per_lane=1, ms=ms)
+                     groups_per_lane=gpl, items_per_lane=1,
+                     one_launch=False, ms=ms)
             trials.append(t)
             if log:
                 log(f"tune {t}")
@@ -97,7 +115,8 @@ def tune(s, reps: int = 3, batches=BATCHES, blocks=BLOCKS,
             s.set_items_per_lane(1)
             t = dict(engine=ENGINE_LEVELS, batches=best["batches"],
                      concurrent=best["concurrent"], block=block,
-                     groups_per_lane=1, items_per_lane=2, ms=ms)
+                     groups_per_lane=1, items_per_lane=2,
+                     one_launch=False, ms=ms)
             trials.append(t)
             if log:
                 log(f"tune {t}")
@@ -119,7 +138,7 @@ def tune(s, reps: int = 3, batches=BATCHES, blocks=BLOCKS,
                          block=level_best["block"],
                          groups_per_lane=level_best["groups_per_lane"],
                          items_per_lane=level_best["items_per_lane"],
-                         chunk_rounds=rounds, ms=ms)
+                         chunk_rounds=rounds, one_launch=False, ms=ms)
                 trials.append(t)
                 if log:
                     log(f"tune {t}")
@@ -140,13 +159,20 @@ def tune(s, reps: int = 3, batches=BATCHES, blocks=BLOCKS,
                      block=level_best["block"],
                      groups_per_lane=level_best["groups_per_lane"],
                      items_per_lane=level_best["items_per_lane"],
-                     chunk_rounds=rounds, priority=tuple(rule), ms=ms)
+                     chunk_rounds=rounds, priority=tuple(rule),
+                     one_launch=False, ms=ms)
             trials.append(t)
             if log:
                 log(f"tune {t}")
             if ms < best["ms"]:
                 best = t
         s.set_priority(*best.get("priority", (-1, 0, 0)))
+    if one and one["ms"] <= best["ms"]:
+        best = one
+        s.set_priority(-1)
+        s.set_launch(best["block"] // ng, 1)
+        s.set_items_per_lane(1)
+        s.set_form(FORM_AUTO)
     s.set_engine(best["engine"], chunk_rounds=best.get("chunk_rounds", 0))
     s.set_schedule(best["batches"])
     s.set_concurrent_batches(best["concurrent"])

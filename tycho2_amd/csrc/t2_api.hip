@@ -61,6 +61,7 @@ struct t2_sweeper {
     int precision = T2_FP64, gauss = T2_GAUSS_NOPIVOT;
     int block = 256, gpl = 1, batches = 1, order = T2_ORDER_FACES;
     int ipl = 1;                     // items per lane (level engine)
+    int form = T2_FORM_AUTO;         // of the level engine's sweeps
     int intra = -1, inter = 0;       // priority schedule (intra < 0: levels)
     int64_t step_width = 0;
     double dep_tol = t2::kTraverseRule;   // dependency rule of the schedule
@@ -292,13 +293,13 @@ int ensure_side_streams(t2_sweeper *s, int64_t n)
 }
 
 // Whether the level engine sweeps with one block per angle: its tables exist
-// and every knob of the step launches is at its default (T2_NO_GRAPH asks
-// for the step launches by name).
+// and nothing asks for the step launches (their knobs, a block size among
+// them, or T2_NO_GRAPH).
 bool angle_form(const t2_sweeper *s)
 {
     return s->angle_gc > 0 && s->engine == T2_ENGINE_LEVELS &&
-           s->batches == 1 && !s->concurrent && s->gpl == 1 && s->ipl == 1 &&
-           s->use_graph;
+           s->form == T2_FORM_AUTO && s->batches == 1 && !s->concurrent &&
+           s->gpl == 1 && s->ipl == 1 && s->use_graph;
 }
 
 t2::AngleSweep angle_tables(const t2_sweeper *s)
@@ -1650,6 +1651,28 @@ int t2_set_launch(t2_sweeper *s, int items_per_block, int groups_per_lane)
     }
     s->block = block;
     s->gpl = gpl;
+    if (items_per_block)   // a shape of the step launches
+        s->form = T2_FORM_STEPS;
+    return T2_OK;
+}
+
+int t2_set_form(t2_sweeper *s, int form)
+{
+    t2::clear_error();
+    if (!s)
+        return fail(T2_ERR_ARG, "null sweeper handle");
+    if (form != T2_FORM_AUTO && form != T2_FORM_STEPS)
+        return fail(T2_ERR_ARG, "form must be T2_FORM_AUTO or T2_FORM_STEPS");
+    s->form = form;
+    return T2_OK;
+}
+
+int t2_get_form(const t2_sweeper *s, int *groups_per_block)
+{
+    t2::clear_error();
+    if (!s || !groups_per_block)
+        return fail(T2_ERR_ARG, "t2_get_form: bad argument");
+    *groups_per_block = angle_form(s) ? s->angle_gc : 0;
     return T2_OK;
 }
 

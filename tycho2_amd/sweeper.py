@@ -29,6 +29,8 @@ ENGINE_QUEUE = 1
 ENGINE_HYBRID = 2
 ORDER_CELL = 0
 ORDER_FACES = 1
+FORM_AUTO = 0
+FORM_STEPS = 1
 ERR_TIMEOUT = -7
 
 _dp = ctypes.POINTER(ctypes.c_double)
@@ -59,6 +61,9 @@ SIGNATURES = {
     "t2_sweeper_info": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p]),
     "t2_set_launch": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int,
                                      ctypes.c_int]),
+    "t2_set_form": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
+    "t2_get_form": (ctypes.c_int, [ctypes.c_void_p,
+                                   ctypes.POINTER(ctypes.c_int)]),
     "t2_set_schedule": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
     "t2_set_order": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
     "t2_set_dependency_tolerance": (ctypes.c_int, [ctypes.c_void_p,
@@ -352,6 +357,17 @@ class SweeperHIP:
     def set_launch(self, items_per_block: int = 0, groups_per_lane: int = 0):
         _check(lib().t2_set_launch(self.handle, items_per_block,
                                    groups_per_lane))
+
+    def set_form(self, form: int) -> None:
+        """FORM_AUTO (one launch where it pays) or FORM_STEPS: the level
+        engine's sweeps.  set_launch with a block size sets FORM_STEPS."""
+        _check(lib().t2_set_form(self.handle, int(form)))
+
+    def form(self) -> int:
+        """Groups a block of the one launch sweeps, 0 for step launches."""
+        gc = ctypes.c_int()
+        _check(lib().t2_get_form(self.handle, ctypes.byref(gc)))
+        return gc.value
 
     def set_items_per_lane(self, items: int) -> None:
         _check(lib().t2_set_items_per_lane(self.handle, int(items)))
