@@ -306,14 +306,17 @@ def batch_leg(args, ev):
                 if t["engine"] == ENGINE_LEVELS:
                     name = (f"levels_c{t['concurrent']}" if t["concurrent"]
                             else "levels")
+                    if t["block"] != autotune.BLOCKS[0]:
+                        name += f"_b{t['block']}"
                 else:
                     name = f"{prefix}_r{t['chunk_rounds']}"
                 out[name] = t["ms"]
+                setting[name] = t
                 log(f"wave {w}: {name} {t['ms']:.2f} ms/sweep, "
                     f"{solves / t['ms'] / 1e6:.1f} G solves/s")
             return out
 
-        timings = {"levels": float("inf")}
+        timings, setting = {"levels": float("inf")}, {}
         with SweepBatch(hs) as b:
             timings.update(tuned(b, "queue", (ENGINE_LEVELS, ENGINE_QUEUE)))
         if rule:
@@ -343,13 +346,7 @@ def batch_leg(args, ev):
         tot["best"] += timings[best]
         tot["solves"] += solves
         with SweepBatch(hs) as b:
-            if best.startswith("levels"):
-                b.set_engine(ENGINE_LEVELS, 0, 0)
-                b.set_concurrent(0 if best == "levels"
-                                 else int(best[len("levels_c"):]))
-            else:
-                b.set_engine(ENGINE_QUEUE, 0,
-                             int(best.rsplit("_r", 1)[1]))
+            autotune.apply_batch(b, setting[best])
             t2 = time.time()
             its, sec = b.solve_krylov(300, 1e-10, 20)
             rec["solve_s"] = round(time.time() - t2, 3)

@@ -163,8 +163,8 @@ int t2_sweeper_create(t2_sweeper **out, int device,
                       const double *sigma_s, int precision, int gauss);
 /* Environment: T2_NO_GRAPH=1 makes the level engine launch its per-step
  * kernels directly, whatever the problem, instead of replaying a captured
- * hipGraph or sweeping in one launch (a debugging aid; results are
- * identical). */
+ * hipGraph or sweeping in one launch; in a batch the handle shares the merged
+ * steps (a debugging aid; results are identical). */
 int t2_sweeper_destroy(t2_sweeper *s);
 int t2_sweeper_info(const t2_sweeper *s, t2_info *info);
 
@@ -407,9 +407,10 @@ int t2_sweep_only(t2_sweeper *s);
  *   T2_ENGINE_LEVELS  members with the same group count share one merged
  *                     step schedule (one launch per merged step and group
  *                     count, replayed from a hipGraph); the merged records
- *                     are a copy of the members' records; members small or
- *                     deep enough for it are swept with one block per angle,
- *                     all of them in one or two launches;
+ *                     are a copy of the members' records; members whose own
+ *                     level sweep would be one launch (t2_get_form) are swept
+ *                     that way, all of them in one or two launches
+ *                     (t2_batch_set_form);
  *   T2_ENGINE_QUEUE   one persistent launch for all members: chunks of the
  *                     members' items interleaved step by step behind one
  *                     ticket counter, each waiting on its own problem's
@@ -430,9 +431,16 @@ int t2_batch_set_engine(t2_batch *b, int engine, int chunk_rounds,
  * on one stream.  Results do not depend on it. */
 int t2_batch_set_concurrent(t2_batch *b, int chains);
 /* Level form: threads per block of the merged step launches (a multiple of
- * 64 in [64, 256]; default 256), one group per lane.  Results do not depend
- * on it (autotuner knob). */
+ * 64 in [64, 256]; default 256), one group per lane; also sets T2_FORM_STEPS.
+ * Results do not depend on it (autotuner knob). */
 int t2_batch_set_launch(t2_batch *b, int block);
+/* Level form: T2_FORM_AUTO (default) sweeps the members that t2_get_form
+ * names with one block per angle, T2_FORM_STEPS all of them in the merged
+ * steps.  A member's own knobs and T2_NO_GRAPH count as they do for the
+ * member alone, whichever engine it is set to.  members_by_angle: how many
+ * members a level-form sweep takes with one block per angle. */
+int t2_batch_set_form(t2_batch *b, int form);
+int t2_batch_get_form(const t2_batch *b, int *members_by_angle);
 /* t2_sweep_step / t2_sweep_only of every member in one batched sweep */
 int t2_batch_sweep_step(t2_batch *b);
 int t2_batch_sweep_only(t2_batch *b);

@@ -18,7 +18,8 @@ Results do not depend on any of these knobs (bitwise, tested).
 """
 from __future__ import annotations
 
-from .sweeper import ENGINE_HYBRID, ENGINE_LEVELS, ENGINE_QUEUE, FORM_AUTO
+from .sweeper import (ENGINE_HYBRID, ENGINE_LEVELS, ENGINE_QUEUE, FORM_AUTO,
+                      FORM_STEPS)
 from .timing import HipEvents, time_region
 
 BATCHES = (1, 2, 4, 8, 16)
@@ -179,23 +180,38 @@ def tune(s, reps: int = 3, batches=BATCHES, blocks=BLOCKS,
     return best, trials
 
 
+def apply_batch(b, t):
+    """Set batch `b` to trial `t` of tune_batch."""
+    b.set_engine(t["engine"], 0, t["chunk_rounds"])
+    b.set_concurrent(t["concurrent"])
+    b.set_launch(t["block"])
+    if t["by_angle"]:
+        b.set_form(FORM_AUTO)
+
+
 def tune_batch(b, reps: int = 3, rounds=CHUNK_ROUNDS,
                engines=(ENGINE_LEVELS, ENGINE_QUEUE), log=None,
                blocks=BLOCKS):
-    """Tune batch `b` in place over its engine (merged per-step launches,
-    their group counts interleaved or on parallel streams, or one
-    persistent ready-queue launch), the level form's block size (at its
-    best chain count) and the queue's chunk size; returns (best, trials)
-    like tune().  A level form that refuses the members' schedules (too
-    many steps) is skipped."""
+    """Tune batch `b` in place over its engine (per-step launches, their
+    group counts interleaved or on parallel streams, or one persistent
+    ready-queue launch), the level form's block size (at its best chain
+    count) and the queue's chunk size; returns (best, trials) like tune().
+    Members that can be swept with one block per angle are (by_angle of a
+    trial counts them) where the chain count is tried, with the others' steps
+    beside them; where there are no others the chains are of no use to it,
+    and only the first trial sweeps that way.  A level form that refuses the
+    members' schedules (too many steps) is skipped."""
     from .sweeper import T2Error
     ev = HipEvents()
     trials = []
 
-    def trial(engine, r, conc, block):
+    def trial(engine, r, conc, block, form):
         b.set_engine(engine, 0, r)
         b.set_concurrent(conc)
         b.set_launch(block)
+        b.set_form(form)
+        t = dict(engine=engine, chunk_rounds=r, concurrent=conc,
+                 block=block, by_angle=b.form())
         try:
             b.sweep_only()
         except T2Error as e:
@@ -203,9 +219,7 @@ def tune_batch(b, reps: int = 3, rounds=CHUNK_ROUNDS,
                 log(f"tune batch engine={engine}: {e}")
             return
         b.synchronize()
-        ms = time_region(ev, b, b.sweep_only, reps) / reps
-        t = dict(engine=engine, chunk_rounds=r, concurrent=conc,
-                 block=block, ms=ms)
+        t["ms"] = time_region(ev, b, b.sweep_only, reps) / reps
         trials.append(t)
         if log:
             log(f"tune batch {t}")
@@ -213,19 +227,21 @@ def tune_batch(b, reps: int = 3, rounds=CHUNK_ROUNDS,
     for engine in engines:
         if engine == ENGINE_QUEUE:
             for r in rounds:
-                trial(engine, r, 0, blocks[0])
+                trial(engine, r, 0, blocks[0], FORM_STEPS)
             continue
+        b.set_engine(engine)
+        b.set_form(FORM_AUTO)
+        alone = b.form() == len(b.members)
         for conc in CHAINS:
-            trial(engine, 0, conc, blocks[0])
+            trial(engine, 0, conc, blocks[0],
+                  FORM_STEPS if alone and conc != CHAINS[0] else FORM_AUTO)
         level = [t for t in trials if t["engine"] == engine]
         if level:
             conc = min(level, key=lambda t: t["ms"])["concurrent"]
             for block in blocks[1:]:
-                trial(engine, 0, conc, block)
+                trial(engine, 0, conc, block, FORM_STEPS)
     if not trials:
         raise RuntimeError("no batch engine could sweep these members")
     best = min(trials, key=lambda t: t["ms"])
-    b.set_engine(best["engine"], 0, best["chunk_rounds"])
-    b.set_concurrent(best["concurrent"])
-    b.set_launch(best["block"])
+    apply_batch(b, best)
     return best, trials

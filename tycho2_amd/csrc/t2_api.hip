@@ -292,14 +292,18 @@ int ensure_side_streams(t2_sweeper *s, int64_t n)
     return T2_OK;
 }
 
-// Whether the level engine sweeps with one block per angle: its tables exist
-// and nothing asks for the step launches (their knobs, a block size among
-// them, or T2_NO_GRAPH).
+// Whether the handle's level sets are swept with one block per angle: its
+// tables exist and nothing asks for the step launches (their knobs, a block
+// size among them, or T2_NO_GRAPH).
+bool angle_levels(const t2_sweeper *s)
+{
+    return s->angle_gc > 0 && s->form == T2_FORM_AUTO && s->batches == 1 &&
+           !s->concurrent && s->gpl == 1 && s->ipl == 1 && s->use_graph;
+}
+
 bool angle_form(const t2_sweeper *s)
 {
-    return s->angle_gc > 0 && s->engine == T2_ENGINE_LEVELS &&
-           s->form == T2_FORM_AUTO && s->batches == 1 && !s->concurrent &&
-           s->gpl == 1 && s->ipl == 1 && s->use_graph;
+    return s->engine == T2_ENGINE_LEVELS && angle_levels(s);
 }
 
 t2::AngleSweep angle_tables(const t2_sweeper *s)
@@ -2361,7 +2365,8 @@ struct t2_batch {
     int engine = T2_ENGINE_LEVELS;
     int concurrent = 0;                  // level form: chains per group count
                                          // (0: all launches on one stream)
-    int block = t2::kMaxBlock;           // level form: threads per block
+    int block = t2::kMaxBlock;           // merged steps: threads per block
+    int form = T2_FORM_AUTO;             // level form: of its members' sweeps
     std::vector<hipStream_t> side;       // their extra streams
     std::vector<hipEvent_t> join_ev;
     hipEvent_t fork_ev = nullptr;
@@ -2373,6 +2378,7 @@ struct t2_batch {
     std::vector<LevelGroup> groups;
     // members swept with one block per angle, in up to two launches (by the
     // LDS their blocks need)
+    std::vector<char> by_angle;          // [members], as the tables were built
     std::vector<int> angle_idx;          // member of each table entry
     void *d_angle_problems = nullptr;    // AngleProblem<T>
     int2 *d_angle_runs = nullptr;
@@ -2408,7 +2414,6 @@ namespace {
 std::vector<const void *> member_buffers(const t2_sweeper *m)
 {
     return {m->d_psi, m->d_src, m->d_sigt, m->d_qang, m->d_pending, m->d_down,
-            m->d_slot_items, m->d_rounds, m->d_angles,
             reinterpret_cast<const void *>(intptr_t(m->generation))};
 }
 
@@ -2659,6 +2664,16 @@ int build_level_group(t2_batch *b, LevelGroup &g)
     return T2_OK;
 }
 
+// Which members the level form sweeps with one block per angle; the others
+// share the merged steps.
+std::vector<char> angle_members(const t2_batch *b)
+{
+    std::vector<char> by_angle;
+    for (const t2_sweeper *m : b->members)
+        by_angle.push_back(b->form == T2_FORM_AUTO && angle_levels(m));
+    return by_angle;
+}
+
 // One-block-per-angle members: their problem table and launches.  Blocks of
 // half the LDS or less run two a CU, the others one: a launch each, the
 // blocks with the most rounds first.
@@ -2673,7 +2688,7 @@ int build_angle_batch(t2_batch *b)
     std::vector<Part> parts;
     for (size_t i = 0; i < b->members.size(); i++) {
         const t2_sweeper *m = b->members[i];
-        if (m->angle_gc <= 0)
+        if (!b->by_angle[i])
             continue;
         const t2::AngleSweep t = angle_tables(m);
         if (!t2::angle_sweep_valid(
@@ -2725,13 +2740,16 @@ int build_angle_batch(t2_batch *b)
 int build_levels(t2_batch *b)
 {
     free_levels(b);
+    b->by_angle = angle_members(b);
     T2_TRY(b->precision == T2_FP64 ? build_angle_batch<double>(b)
                                    : build_angle_batch<float>(b));
     std::vector<int> ngs;
-    for (auto *m : b->members)
-        if (m->angle_gc <= 0 &&
-            std::find(ngs.begin(), ngs.end(), int(m->ng)) == ngs.end())
-            ngs.push_back(int(m->ng));
+    for (size_t i = 0; i < b->members.size(); i++) {
+        const int ng = int(b->members[i]->ng);
+        if (!b->by_angle[i] &&
+            std::find(ngs.begin(), ngs.end(), ng) == ngs.end())
+            ngs.push_back(ng);
+    }
     std::sort(ngs.begin(), ngs.end());
     // one merged schedule per group count, or, for parallel chains, up to
     // `concurrent` per group count with the members dealt out by work
@@ -2740,7 +2758,7 @@ int build_levels(t2_batch *b)
     for (int ng : ngs) {
         std::vector<int> idx;
         for (size_t i = 0; i < b->members.size(); i++)
-            if (b->members[i]->angle_gc <= 0 && b->members[i]->ng == ng)
+            if (!b->by_angle[i] && b->members[i]->ng == ng)
                 idx.push_back(int(i));
         auto work = [&](int i) {
             return b->members[i]->nc * b->members[i]->na * b->members[i]->ng;
@@ -2950,7 +2968,8 @@ int batch_sweep(t2_batch *b)
                                        : build_batch_queue<float>(b));
         batch_snapshot(b);
     }
-    if (b->engine == T2_ENGINE_LEVELS && !b->levels_built) {
+    if (b->engine == T2_ENGINE_LEVELS &&
+        (!b->levels_built || b->by_angle != angle_members(b))) {
         // one launch per merged step and group count
         std::vector<std::pair<int64_t, int64_t>> longest;  // (groups, steps)
         for (auto *m : b->members) {
@@ -3166,12 +3185,37 @@ int t2_batch_set_launch(t2_batch *b, int block)
     if (block < 64 || block > t2::kMaxBlock || block % 64)
         return fail(T2_ERR_ARG, "block must be a multiple of 64 in [64, " +
                                     std::to_string(t2::kMaxBlock) + "]");
+    b->form = T2_FORM_STEPS;   // a shape of the merged steps
     if (block == b->block)
         return T2_OK;
     T2_HIP(hipSetDevice(b->device));
     T2_HIP(hipStreamSynchronize(b->stream));
     drop_batch_graph(b);
     b->block = block;
+    return T2_OK;
+}
+
+int t2_batch_set_form(t2_batch *b, int form)
+{
+    t2::clear_error();
+    if (!b)
+        return fail(T2_ERR_ARG, "null batch");
+    if (form != T2_FORM_AUTO && form != T2_FORM_STEPS)
+        return fail(T2_ERR_ARG, "form must be T2_FORM_AUTO or T2_FORM_STEPS");
+    b->form = form;
+    return T2_OK;
+}
+
+int t2_batch_get_form(const t2_batch *b, int *members_by_angle)
+{
+    t2::clear_error();
+    if (!b || !members_by_angle)
+        return fail(T2_ERR_ARG, "t2_batch_get_form: bad argument");
+    const std::vector<char> by_angle = angle_members(b);
+    *members_by_angle =
+        b->engine == T2_ENGINE_LEVELS
+            ? int(std::count(by_angle.begin(), by_angle.end(), 1))
+            : 0;
     return T2_OK;
 }
 

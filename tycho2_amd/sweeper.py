@@ -120,6 +120,9 @@ SIGNATURES = {
     "t2_batch_set_concurrent": (ctypes.c_int, [ctypes.c_void_p,
                                                ctypes.c_int]),
     "t2_batch_set_launch": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
+    "t2_batch_set_form": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
+    "t2_batch_get_form": (ctypes.c_int, [ctypes.c_void_p,
+                                         ctypes.POINTER(ctypes.c_int)]),
     "t2_batch_sweep_step": (ctypes.c_int, [ctypes.c_void_p]),
     "t2_batch_sweep_only": (ctypes.c_int, [ctypes.c_void_p]),
     "t2_batch_info": (ctypes.c_int, [ctypes.c_void_p, _ip, _ip]),
@@ -587,8 +590,20 @@ class SweepBatch:
                                          int(chunk_rounds), int(spin_limit)))
 
     def set_launch(self, block: int) -> None:
-        """Threads per block of the level form's merged launches."""
+        """Threads per block of the level form's merged launches (sets
+        FORM_STEPS)."""
         _check(lib().t2_batch_set_launch(self.handle, int(block)))
+
+    def set_form(self, form: int) -> None:
+        """Level form: FORM_AUTO sweeps the members whose own level sweep is
+        one launch that way, FORM_STEPS all of them in merged steps."""
+        _check(lib().t2_batch_set_form(self.handle, int(form)))
+
+    def form(self) -> int:
+        """Members that a level-form sweep takes with one block per angle."""
+        n = ctypes.c_int()
+        _check(lib().t2_batch_get_form(self.handle, ctypes.byref(n)))
+        return n.value
 
     def set_concurrent(self, chains: int) -> None:
         """Level form: independent merged schedules on parallel streams,
