@@ -45,7 +45,7 @@ extern "C" {
 #define T2_ERR_STATE -4    /* call not valid in the handle's current state */
 #define T2_ERR_NODEV -5    /* no usable GPU                                */
 #define T2_ERR_NOCONV -6   /* iteration hit its limit without converging   */
-#define T2_ERR_TIMEOUT -7  /* a ready-queue wait ran past its poll limit   */
+#define T2_ERR_TIMEOUT -7  /* a wait inside a sweep ran past its limit     */
 
 /* sweep arithmetic (also the angular-flux storage type) */
 #define T2_FP64 0
@@ -184,6 +184,12 @@ int t2_set_form(t2_sweeper *s, int form);
 /* Groups a block of the one launch sweeps, 0 where a level-engine sweep of
  * the handle, as it is set now, makes step launches. */
 int t2_get_form(const t2_sweeper *s, int *groups_per_block);
+/* Bounds each wait inside the one launch (polls of some 0.4 us; 0 = default,
+ * seconds, far beyond any wait of a correct sweep).  A wait that runs out
+ * abandons the sweep, and the next synchronising call on the handle (or on
+ * the batch that swept it; a batch takes its members' smallest limit) returns
+ * T2_ERR_TIMEOUT; later sweeps are valid. */
+int t2_set_wait_limit(t2_sweeper *s, int64_t polls);
 
 /* Items per lane of the level engine's step launches (1 or 2; NoPivot cell
  * solver and one group per lane only): with 2 a wavefront solves two sets

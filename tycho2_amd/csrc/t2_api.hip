@@ -52,6 +52,12 @@ struct GraphEntry {
     hipGraphExec_t exec;
 };
 
+// The flag of abandoned one-launch sweeps: host memory that the GPU writes, so
+// that reading it costs a call nothing once its stream is idle.
+struct StallFlag {
+    int32_t *host = nullptr, *device = nullptr;
+};
+
 }  // namespace
 
 struct t2_sweeper {
@@ -101,6 +107,8 @@ struct t2_sweeper {
     t2::AngleRound *d_rounds = nullptr;
     int32_t *d_angles = nullptr;     // round_off [na + 1], order [na],
                                      // lag_off [na + 1]
+    StallFlag stalled;               // its abandoned sweeps
+    int64_t wait_limit = 0;          // polls (0: default)
     // fluxes and sources
     void *d_psi = nullptr;           // T [na][nc][4][G]
     void *d_src = nullptr;           // T [nc][4][G]
@@ -323,6 +331,35 @@ t2::AngleSweep angle_tables(const t2_sweeper *s)
     return t;
 }
 
+int ensure_stall_flag(StallFlag *f)
+{
+    if (f->host)
+        return T2_OK;
+    int32_t *h = nullptr;
+    T2_HIP(hipHostMalloc(reinterpret_cast<void **>(&h), sizeof(int32_t),
+                         hipHostMallocMapped | hipHostMallocCoherent));
+    *h = 0;
+    f->host = h;
+    T2_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&f->device), h,
+                                   0));
+    return T2_OK;
+}
+
+t2::AngleGuard angle_guard(const StallFlag &f, int64_t limit)
+{
+    return {f.device, limit > 0 ? uint32_t(limit) : t2::kMaxPolls};
+}
+
+// Reports an abandoned one-launch sweep once (its stream is idle).
+int check_stalled(const StallFlag &f)
+{
+    if (!f.host || !__atomic_exchange_n(f.host, 0, __ATOMIC_ACQ_REL))
+        return T2_OK;
+    return fail(T2_ERR_TIMEOUT,
+                "a wait of a one-launch sweep ran past its poll limit; the "
+                "sweep was abandoned and its results are invalid");
+}
+
 // Step launches store psi past the caches when an average step writes more
 // of it than kCachedStep: a step reads about three times what it writes, and
 // its cells are read for a few steps after it, so beyond about a sixteenth of
@@ -386,8 +423,9 @@ int enqueue_sweep(t2_sweeper *s, const double *ang, const void *ang_t,
         a.geo = geo;
         a.topo = s->d_item_topo;
         a.n_items = s->nc * s->na;
-        T2_HIP(t2::launch_angle_sweep<T>(a, angle_tables(s), s->angle_block,
-                                         s->stream));
+        T2_HIP(t2::launch_angle_sweep<T>(
+            a, angle_tables(s), angle_guard(s->stalled, s->wait_limit),
+            s->angle_block, s->stream));
         return T2_OK;
     }
     const int64_t nb = int64_t(s->sched.batch_steps.size()) - 1;
@@ -577,10 +615,12 @@ int ensure_queue(t2_sweeper *s)
     return build_queue(s, first);
 }
 
-// After an abandoned ready-queue sweep: reports it once and re-arms the
-// counters so that later sweeps are valid.
+// After an abandoned sweep, with the stream idle or a ready queue to wait for:
+// reports it once and re-arms the queue's counters so that later sweeps are
+// valid.
 int check_abort(t2_sweeper *s)
 {
+    T2_TRY(check_stalled(s->stalled));
     if (!s->d_abort)
         return T2_OK;
     int32_t flag = 0;
@@ -1030,6 +1070,7 @@ int build_angle_tables(t2_sweeper *s)
     std::copy(lag_off.begin(), lag_off.end(), order + na);
     const size_t n_items = size_t(nc) * na;
     s->n_rounds = int64_t(rounds.size());
+    T2_TRY(ensure_stall_flag(&s->stalled));
     uint16_t *d_slot = nullptr;
     T2_TRY(dalloc_t(s, &d_slot, sizeof(uint16_t) * n_items));
     int rc = T2_OK;
@@ -1581,6 +1622,8 @@ int t2_sweeper_destroy(t2_sweeper *s)
         if (s->pin_ev[b])
             (void)hipEventDestroy(s->pin_ev[b]);
     }
+    if (s->stalled.host)
+        (void)hipHostFree(s->stalled.host);
     for (size_t i = 0; i < s->side.size(); i++) {
         (void)hipStreamSynchronize(s->side[i]);
         (void)hipStreamDestroy(s->side[i]);
@@ -1677,6 +1720,17 @@ int t2_get_form(const t2_sweeper *s, int *groups_per_block)
     if (!s || !groups_per_block)
         return fail(T2_ERR_ARG, "t2_get_form: bad argument");
     *groups_per_block = angle_form(s) ? s->angle_gc : 0;
+    return T2_OK;
+}
+
+int t2_set_wait_limit(t2_sweeper *s, int64_t polls)
+{
+    t2::clear_error();
+    if (!s)
+        return fail(T2_ERR_ARG, "null sweeper handle");
+    if (polls < 0 || polls > int64_t(INT32_MAX))
+        return fail(T2_ERR_ARG, "polls must be in [0, 2^31)");
+    s->wait_limit = polls;
     return T2_OK;
 }
 
@@ -2069,7 +2123,8 @@ int t2_get_psi(const t2_sweeper *s_const, double *psi)
         T2_HIP(t2::launch_ac_to_ca<float>(
             static_cast<const float *>(s->d_psi), s->d_stage, s->nc, s->na,
             4 * s->ng, s->stream, s->psi_corrected ? s->d_res : nullptr));
-    return download_host(s, psi, s->d_stage, sizeof(double) * n);
+    T2_TRY(download_host(s, psi, s->d_stage, sizeof(double) * n));
+    return check_stalled(s->stalled);
 }
 
 int t2_defect(t2_sweeper *s, const double *psi, double *density)
@@ -2139,7 +2194,8 @@ int t2_defect(t2_sweeper *s, const double *psi, double *density)
         T2_HIP(t2::launch_ac_to_ca<float>(s->d_res, s->d_stage, s->nc, s->na,
                                           vg, s->stream));
     }
-    return download_host(s, density, s->d_stage, sizeof(double) * n);
+    T2_TRY(download_host(s, density, s->d_stage, sizeof(double) * n));
+    return check_stalled(s->stalled);
 }
 
 static int krylov_vectors(t2_sweeper *s)
@@ -2226,7 +2282,7 @@ int t2_get_psi_angle(const t2_sweeper *s, int64_t angle, double *psi_a)
         for (int64_t i = 0; i < n; i++)
             psi_a[i] = double(tmp[i]) + (corr.empty() ? 0.0 : double(corr[i]));
     }
-    return T2_OK;
+    return check_stalled(s->stalled);
 }
 
 int t2_synchronize(t2_sweeper *s)
@@ -2378,7 +2434,9 @@ struct t2_batch {
     std::vector<LevelGroup> groups;
     // members swept with one block per angle, in up to two launches (by the
     // LDS their blocks need)
-    std::vector<char> by_angle;          // [members], as the tables were built
+    std::vector<int64_t> by_angle;       // [members], as the tables were
+                                         // built: 0 no, else 1 + wait limit
+    StallFlag stalled;                   // their abandoned sweeps
     std::vector<int> angle_idx;          // member of each table entry
     void *d_angle_problems = nullptr;    // AngleProblem<T>
     int2 *d_angle_runs = nullptr;
@@ -2666,11 +2724,13 @@ int build_level_group(t2_batch *b, LevelGroup &g)
 
 // Which members the level form sweeps with one block per angle; the others
 // share the merged steps.
-std::vector<char> angle_members(const t2_batch *b)
+std::vector<int64_t> angle_members(const t2_batch *b)
 {
-    std::vector<char> by_angle;
+    std::vector<int64_t> by_angle;
     for (const t2_sweeper *m : b->members)
-        by_angle.push_back(b->form == T2_FORM_AUTO && angle_levels(m));
+        by_angle.push_back(b->form == T2_FORM_AUTO && angle_levels(m)
+                               ? 1 + m->wait_limit
+                               : 0);
     return by_angle;
 }
 
@@ -2701,6 +2761,7 @@ int build_angle_batch(t2_batch *b)
     }
     if (parts.empty())
         return T2_OK;
+    T2_TRY(ensure_stall_flag(&b->stalled));
     auto big = [](const Part &p) { return p.lds > t2::kMaxLds / 2; };
     std::stable_sort(parts.begin(), parts.end(),
                      [&](const Part &x, const Part &y) {
@@ -2881,11 +2942,19 @@ int batch_enqueue(t2_batch *b)
     }
     // all members carry an angle-dependent source or none does
     auto launch_angles = [&]() {
+        if (b->angle_launches.empty())
+            return T2_OK;
+        int64_t limit = 0;               // the members' smallest
+        for (int64_t l : b->by_angle)
+            if (l > 1 && (limit == 0 || l - 1 < limit))
+                limit = l - 1;
+        const t2::AngleGuard guard = angle_guard(b->stalled, limit);
         for (const auto &l : b->angle_launches)
             T2_HIP(t2::launch_angle_batch<T>(
                 static_cast<const t2::AngleProblem<T> *>(b->d_angle_problems),
                 b->d_angle_runs + l.first_run, l.n_runs, l.n_blocks,
-                b->d_angle_active, b->ang_t[0] != nullptr, l.lds, b->stream));
+                b->d_angle_active, guard, b->ang_t[0] != nullptr, l.lds,
+                b->stream));
         return T2_OK;
     };
     auto launch = [&](LevelGroup &g, int64_t st, hipStream_t stream) {
@@ -3064,14 +3133,17 @@ int batch_sweep(t2_batch *b)
     return T2_OK;
 }
 
-// After an abandoned batched ready-queue sweep: reports it once and re-arms
-// every member's counters.
+// After an abandoned batched sweep: reports it once and re-arms every member's
+// ready-queue counters.
 int batch_check_abort(t2_batch *b)
 {
+    if (!b->stalled.host && !b->d_abort)
+        return T2_OK;
+    T2_HIP(hipStreamSynchronize(b->stream));
+    T2_TRY(check_stalled(b->stalled));
     if (!b->d_abort)
         return T2_OK;
     int32_t flag = 0;
-    T2_HIP(hipStreamSynchronize(b->stream));
     T2_HIP(hipMemcpy(&flag, b->d_abort, sizeof(flag), hipMemcpyDeviceToHost));
     if (!flag)
         return T2_OK;
@@ -3160,6 +3232,8 @@ int t2_batch_destroy(t2_batch *b)
         (void)hipFree(b->d_ticket);
     if (b->d_abort)
         (void)hipFree(b->d_abort);
+    if (b->stalled.host)
+        (void)hipHostFree(b->stalled.host);
     if (b->d_active)
         (void)hipFree(b->d_active);
     if (b->order)
@@ -3211,10 +3285,11 @@ int t2_batch_get_form(const t2_batch *b, int *members_by_angle)
     t2::clear_error();
     if (!b || !members_by_angle)
         return fail(T2_ERR_ARG, "t2_batch_get_form: bad argument");
-    const std::vector<char> by_angle = angle_members(b);
+    const std::vector<int64_t> by_angle = angle_members(b);
     *members_by_angle =
         b->engine == T2_ENGINE_LEVELS
-            ? int(std::count(by_angle.begin(), by_angle.end(), 1))
+            ? int(by_angle.size() -
+                  size_t(std::count(by_angle.begin(), by_angle.end(), 0)))
             : 0;
     return T2_OK;
 }

@@ -176,6 +176,15 @@ struct AngleSweep {
     int chunks;                    // blocks per angle (groups split evenly)
 };
 
+// Bound of a block's waits: past max_polls polls (of eight looks at an LDS
+// counter, some 0.4 us) a wavefront gives the sweep up, runs on without
+// waiting and raises the flag (host memory).
+constexpr uint32_t kMaxPolls = 1u << 23;   // seconds
+struct AngleGuard {
+    int32_t *stalled;
+    uint32_t max_polls;            // below 2^31
+};
+
 // LDS of a block: its count and a table of `slots` slots for gc groups.
 inline size_t angle_lds_bytes(int64_t slots, int gc, size_t value)
 {
@@ -184,7 +193,8 @@ inline size_t angle_lds_bytes(int64_t slots, int gc, size_t value)
 
 template <typename T>
 hipError_t launch_angle_sweep(const SweepArgs<T> &args, const AngleSweep &t,
-                              int block, hipStream_t stream);
+                              const AngleGuard &guard, int block,
+                              hipStream_t stream);
 // Blocks of a sweep: a multiple of 8 (one XCD per angle's chunks).
 inline int angle_blocks(const AngleSweep &t)
 {
@@ -205,8 +215,8 @@ struct AngleProblem {
 template <typename T>
 hipError_t launch_angle_batch(const AngleProblem<T> *problems,
                               const int2 *runs, int n_runs, int n_blocks,
-                              const int32_t *active, bool ang_t, size_t lds,
-                              hipStream_t stream);
+                              const int32_t *active, const AngleGuard &guard,
+                              bool ang_t, size_t lds, hipStream_t stream);
 
 hipError_t launch_slot_items(const ItemTopo *topo, const uint16_t *slot,
                              const int32_t *lag_off, int n_slots, int zero,

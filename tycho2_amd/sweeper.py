@@ -64,6 +64,7 @@ SIGNATURES = {
     "t2_set_form": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
     "t2_get_form": (ctypes.c_int, [ctypes.c_void_p,
                                    ctypes.POINTER(ctypes.c_int)]),
+    "t2_set_wait_limit": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int64]),
     "t2_set_schedule": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
     "t2_set_order": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
     "t2_set_dependency_tolerance": (ctypes.c_int, [ctypes.c_void_p,
@@ -371,6 +372,10 @@ class SweeperHIP:
         gc = ctypes.c_int()
         _check(lib().t2_get_form(self.handle, ctypes.byref(gc)))
         return gc.value
+
+    def set_wait_limit(self, polls: int) -> None:
+        """Bound of each wait inside the one launch, in polls (0: default)."""
+        _check(lib().t2_set_wait_limit(self.handle, int(polls)))
 
     def set_items_per_lane(self, items: int) -> None:
         _check(lib().t2_set_items_per_lane(self.handle, int(items)))
