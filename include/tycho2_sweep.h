@@ -177,7 +177,9 @@ int t2_set_launch(t2_sweeper *s, int items_per_block, int groups_per_lane);
  * problems in one launch, a block sweeping an angle through its levels, while
  * the knobs of the step launches (groups and items per lane, angle batches)
  * are at their defaults; T2_FORM_STEPS: one launch per schedule step whatever
- * the problem.  Results are bitwise the same. */
+ * the problem.  Results are bitwise the same.  Where the device has no memory
+ * for the one launch's tables, or a later call needs theirs, the handle makes
+ * step launches until its schedule is next rebuilt. */
 #define T2_FORM_AUTO 0
 #define T2_FORM_STEPS 1
 int t2_set_form(t2_sweeper *s, int form);

@@ -157,11 +157,11 @@ namespace {
 // brings the count down to zero fails as an out-of-memory would.
 std::atomic<int64_t> g_alloc_fail{0};
 
-int dalloc(t2_sweeper *s, void **p, size_t bytes)
+void free_angle_form(t2_sweeper *s);
+
+int dalloc_once(t2_sweeper *s, void **p, size_t bytes)
 {
     *p = nullptr;
-    if (bytes == 0)
-        bytes = 8;
     if (g_alloc_fail.load(std::memory_order_relaxed) > 0 &&
         --g_alloc_fail == 0)
         return fail(T2_ERR_NOMEM, "hipMalloc(" + std::to_string(bytes) +
@@ -176,6 +176,23 @@ int dalloc(t2_sweeper *s, void **p, size_t bytes)
     s->allocs.push_back(*p);
     s->bytes += bytes;
     return T2_OK;
+}
+
+// Where the device runs out of memory the one-launch form's tables make room:
+// the step launches need none of them.  (A batch that sweeps the handle has
+// been ordered before the handle's stream, and looks at its members' forms
+// before each sweep.)
+int dalloc(t2_sweeper *s, void **p, size_t bytes)
+{
+    if (bytes == 0)
+        bytes = 8;
+    const int rc = dalloc_once(s, p, bytes);
+    if (rc != T2_ERR_NOMEM || s->angle_gc == 0)
+        return rc;
+    T2_HIP(hipStreamSynchronize(s->stream));
+    free_angle_form(s);
+    t2::clear_error();
+    return dalloc_once(s, p, bytes);
 }
 
 template <typename P>
@@ -1019,7 +1036,7 @@ int build_angle_tables(t2_sweeper *s)
 {
     const int64_t nc = s->nc, na = s->na;
     const auto &sc = s->sched;
-    if (sc.slice.empty() || s->batches != 1 ||
+    if (sc.slice.empty() || s->batches != 1 || !s->use_graph ||
         s->gauss != T2_GAUSS_NOPIVOT ||
         s->n_phi() * int64_t(sizeof(double)) >= (int64_t(1) << 32))
         return T2_OK;
@@ -1138,7 +1155,7 @@ void free_schedule(t2_sweeper *s)
 }
 
 // Level sets, lagged faces and item records for the current batch count.
-int build_schedule_device(t2_sweeper *s)
+int build_records(t2_sweeper *s)
 {
     const int64_t nc = s->nc, na = s->na, ng = s->ng;
     free_schedule(s);
@@ -1220,10 +1237,21 @@ int build_schedule_device(t2_sweeper *s)
                                      s->d_item_geo64);
     }
     cleanup();
-    if (rc == T2_OK)
-        rc = build_angle_form(s);
+    return rc;
+}
+
+// ... and, last of all a handle allocates, the one-launch form's tables.
+int finish_schedule(t2_sweeper *s)
+{
+    const int rc = build_angle_form(s);
     std::vector<uint32_t>().swap(s->sched.work);
     return rc;
+}
+
+int build_schedule_device(t2_sweeper *s)
+{
+    T2_TRY(build_records(s));
+    return finish_schedule(s);
 }
 
 int setup_device(t2_sweeper *s, const double *weights, const double *sigma_s)
@@ -1264,7 +1292,7 @@ int setup_device(t2_sweeper *s, const double *weights, const double *sigma_s)
     }
     T2_TRY(dalloc_t(s, &s->d_nbr, sizeof(uint32_t) * nc));
     T2_TRY(upload(s->d_nbr, s->hm.nbr_pack.data(), nc));
-    T2_TRY(build_schedule_device(s));
+    T2_TRY(build_records(s));
 
     T2_TRY(dalloc(s, &s->d_psi, ts * size_t(na) * n_phi));
     T2_TRY(dalloc(s, &s->d_src, ts * size_t(n_phi)));
@@ -1272,6 +1300,7 @@ int setup_device(t2_sweeper *s, const double *weights, const double *sigma_s)
     T2_TRY(dalloc_t(s, &s->d_phi_old, sizeof(double) * n_phi));
     T2_TRY(dalloc_t(s, &s->d_red, sizeof(double) * t2::kRedBlocks * 64));
     T2_TRY(dalloc_t(s, &s->d_scal, sizeof(double) * t2::kArnoldiScalars));
+    T2_TRY(finish_schedule(s));
     T2_TRY(zero_psi(s));
     T2_TRY(total_source(s, nullptr, nullptr));
     T2_HIP(t2::launch_fill(s->d_phi, 0.0, n_phi, s->stream));
