@@ -8,6 +8,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -1121,7 +1122,12 @@ int build_angle_tables(t2_sweeper *s)
 // the handle keeps to the step launches.
 int build_angle_form(t2_sweeper *s)
 {
-    const int rc = build_angle_tables(s);
+    int rc = T2_OK;
+    try {
+        rc = build_angle_tables(s);
+    } catch (const std::bad_alloc &) {
+        rc = fail(T2_ERR_NOMEM, "host memory for the sweep's tables");
+    }
     if (rc == T2_OK && s->angle_gc > 0)
         return T2_OK;
     free_angle_form(s);

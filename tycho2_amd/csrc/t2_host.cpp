@@ -5,6 +5,7 @@
 #include <array>
 #include <atomic>
 #include <cmath>
+#include <new>
 #include <random>
 #include <thread>
 
@@ -259,22 +260,47 @@ static int n_workers(int64_t jobs)
 
 namespace {
 
+// Runs work(w) on nw host threads.  What one of them throws would end the
+// process there: it is thrown here instead, once all have ended.  Fewer
+// threads than asked for will do (they take their jobs from one counter).
+template <typename F>
+void run_workers(int nw, F work)
+{
+    std::atomic<bool> failed{false};
+    auto guarded = [&](int w) {
+        try {
+            work(w);
+        } catch (...) {
+            failed = true;
+        }
+    };
+    std::vector<std::thread> pool;
+    try {
+        for (int w = 1; w < nw; w++)
+            pool.emplace_back(guarded, w);
+    } catch (...) {
+    }
+    guarded(0);
+    for (auto &t : pool)
+        t.join();
+    if (failed)
+        throw std::bad_alloc();
+}
+
 // Runs body(a) for every angle on the host's cores.
 template <typename F>
 void for_each_angle(int64_t na, F body)
 {
-    const int nw = n_workers(na);
     std::atomic<int64_t> next{0};
-    auto work = [&]() {
+    run_workers(n_workers(na), [&](int) {
         for (int64_t a; (a = next.fetch_add(1)) < na;)
             body(a);
-    };
-    std::vector<std::thread> pool;
-    for (int w = 1; w < nw; w++)
-        pool.emplace_back(work);
-    work();
-    for (auto &t : pool)
-        t.join();
+    });
+}
+
+int no_host_memory()
+{
+    return fail(T2_ERR_NOMEM, "host memory for the sweep schedule");
 }
 
 }  // namespace
@@ -282,22 +308,16 @@ void for_each_angle(int64_t na, F body)
 int build_levels(const HostMesh &m, int64_t na, const double *omega,
                  int32_t *levels, std::vector<LaggedFace> &lagged,
                  double dep_tol)
-{
+try {
     const int nw = n_workers(na);
     std::vector<std::vector<LaggedFace>> lag(nw);
     std::atomic<int64_t> next{0};
-    auto work = [&](int w) {
+    run_workers(nw, [&](int w) {
         std::vector<int32_t> indeg, frontier;
         for (int64_t a; (a = next.fetch_add(1)) < na;)
             angle_levels(m, omega + 3 * a, int32_t(a), levels + a * m.nc,
                          lag[w], indeg, frontier, dep_tol);
-    };
-    std::vector<std::thread> pool;
-    for (int w = 1; w < nw; w++)
-        pool.emplace_back(work, w);
-    work(0);
-    for (auto &t : pool)
-        t.join();
+    });
     lagged.clear();
     for (auto &l : lag)
         lagged.insert(lagged.end(), l.begin(), l.end());
@@ -308,6 +328,8 @@ int build_levels(const HostMesh &m, int64_t na, const double *omega,
                   return x.face < y.face;
               });
     return T2_OK;
+} catch (const std::bad_alloc &) {
+    return no_host_memory();
 }
 
 std::vector<int32_t> angle_batches(int64_t na, const double *omega,
@@ -393,7 +415,7 @@ static void level_after_lagging(const HostMesh &m, const double *omega,
 // (angle, cell) of the batch at level l, angle-major and cell-ascending.
 int build_schedule(const HostMesh &m, int64_t na, const double *omega,
                    int batches, int order, Schedule &s, double dep_tol)
-{
+try {
     const int64_t nc = m.nc;
     int cb = 1;
     while ((int64_t(1) << cb) < nc)
@@ -486,6 +508,8 @@ int build_schedule(const HostMesh &m, int64_t na, const double *omega,
                             sl[lev].first;
     }
     return T2_OK;
+} catch (const std::bad_alloc &) {
+    return no_host_memory();
 }
 
 // ------------------------------------------------------------ priorities
@@ -500,15 +524,11 @@ int build_schedule(const HostMesh &m, int64_t na, const double *omega,
 int build_slots(const HostMesh &m, int64_t na, const double *omega,
                 const Schedule &s, std::vector<uint16_t> &slot,
                 int64_t *n_slots)
-{
+try {
     constexpr int32_t kHandedOn = -2;
     const int64_t nc = m.nc;
     const uint32_t cmask = (uint32_t(1) << s.cell_bits) - 1;
-    try {
-        slot.assign(size_t(na) * nc, kNoSlot);
-    } catch (...) {
-        return fail(T2_ERR_NOMEM, "host memory for the sweep's slots");
-    }
+    slot.assign(size_t(na) * nc, kNoSlot);
     std::vector<int64_t> most(na, 0);
     for_each_angle(na, [&](int64_t a) {
         const double *om = omega + 3 * a;
@@ -578,6 +598,8 @@ int build_slots(const HostMesh &m, int64_t na, const double *omega,
     });
     *n_slots = *std::max_element(most.begin(), most.end());
     return T2_OK;
+} catch (const std::bad_alloc &) {
+    return no_host_memory();
 }
 
 namespace {
@@ -666,7 +688,7 @@ int sweep_priorities(const HostMesh &m, int64_t na, const double *omega,
                      const int32_t *levels,
                      const std::vector<LaggedFace> &lagged, int intra,
                      int inter, std::vector<uint64_t> &prio)
-{
+try {
     if (intra < 0 || intra > 4 || inter < 0 || inter > 2)
         return fail(T2_ERR_ARG, "intraAngleP must be in [0, 4] and "
                                 "interAngleP in [0, 2]");
@@ -755,13 +777,15 @@ int sweep_priorities(const HostMesh &m, int64_t na, const double *omega,
         }
     }
     return T2_OK;
+} catch (const std::bad_alloc &) {
+    return no_host_memory();
 }
 
 int build_priority_schedule(const HostMesh &m, int64_t na,
                             const double *omega, int intra, int inter,
                             int64_t width, int order, Schedule &s,
                             double dep_tol)
-{
+try {
     const int64_t nc = m.nc;
     int cb = 1;
     while ((int64_t(1) << cb) < nc)
@@ -884,6 +908,8 @@ int build_priority_schedule(const HostMesh &m, int64_t na,
     s.lev_off.clear();
     s.slice.clear();
     return T2_OK;
+} catch (const std::bad_alloc &) {
+    return no_host_memory();
 }
 
 }  // namespace t2
