@@ -376,13 +376,13 @@ static void level_after_lagging(const HostMesh &m, const double *omega,
         const int64_t a = lagged[runs[r].first].angle;
         const double *om = omega + 3 * a;
         int32_t *level = levels + a * nc;
-        std::vector<uint8_t> lag(nc, 0), left(nc, 0);
+        std::vector<uint8_t> met(nc, 0), left(nc, 0);   // lagged or released
         for (size_t i = runs[r].first; i < runs[r].second; i++)
-            lag[lagged[i].cell] |= uint8_t(1u << lagged[i].face);
+            met[lagged[i].cell] |= uint8_t(1u << lagged[i].face);
         std::vector<int32_t> front, next;
         for (int64_t c = 0; c < nc; c++) {
             for (int k = 0; k < 4; k++)
-                left[c] += m.adj[4 * c + k] >= 0 && !(lag[c] >> k & 1u) &&
+                left[c] += m.adj[4 * c + k] >= 0 && !(met[c] >> k & 1u) &&
                            !(omega_dot_n(om, &m.normal[(4 * c + k) * 3]) > 0);
             if (!left[c])
                 front.push_back(int32_t(c));
@@ -399,9 +399,12 @@ static void level_after_lagging(const HostMesh &m, const double *omega,
                     int back = 0;  // u's face towards c
                     while (m.adj[4 * u + back] != c)
                         back++;
-                    if (!(lag[u] >> back & 1u) &&
-                        !(omega_dot_n(om, &m.normal[(4 * u + back) * 3]) > 0) &&
-                        --left[u] == 0)
+                    if ((met[u] >> back & 1u) ||
+                        omega_dot_n(om, &m.normal[(4 * u + back) * 3]) > 0)
+                        continue;
+                    // once, also where the cells share another face
+                    met[u] |= uint8_t(1u << back);
+                    if (--left[u] == 0)
                         next.push_back(int32_t(u));
                 }
             }
