@@ -287,12 +287,15 @@ void run_workers(int nw, F work)
         throw std::bad_alloc();
 }
 
-// Runs body(a) for every angle on the host's cores.
+// Runs body(a) for every angle on the host's cores, a thread for every `grain`
+// of the items (a thread takes some 6 us to start).
+constexpr int64_t kGrain = 2000;         // of tens of ns an item
+constexpr int64_t kListGrain = 8000;     // of a few
 template <typename F>
-void for_each_angle(int64_t na, F body)
+void for_each_angle(int64_t na, int64_t items, int64_t grain, F body)
 {
     std::atomic<int64_t> next{0};
-    run_workers(n_workers(na), [&](int) {
+    run_workers(n_workers(std::min(na, items / grain)), [&](int) {
         for (int64_t a; (a = next.fetch_add(1)) < na;)
             body(a);
     });
@@ -309,7 +312,7 @@ int build_levels(const HostMesh &m, int64_t na, const double *omega,
                  int32_t *levels, std::vector<LaggedFace> &lagged,
                  double dep_tol)
 try {
-    const int nw = n_workers(na);
+    const int nw = n_workers(std::min(na, m.nc * na / kGrain));
     std::vector<std::vector<LaggedFace>> lag(nw);
     std::atomic<int64_t> next{0};
     run_workers(nw, [&](int w) {
@@ -372,7 +375,8 @@ static void level_after_lagging(const HostMesh &m, const double *omega,
         runs.push_back({i, j});
         i = j;
     }
-    for_each_angle(int64_t(runs.size()), [&](int64_t r) {
+    for_each_angle(int64_t(runs.size()), nc * int64_t(runs.size()), kGrain,
+                   [&](int64_t r) {
         const int64_t a = lagged[runs[r].first].angle;
         const double *om = omega + 3 * a;
         int32_t *level = levels + a * nc;
@@ -442,16 +446,24 @@ try {
     level_after_lagging(m, omega, s.lagged, levels.data());
     const std::vector<int32_t> batch = angle_batches(na, omega, batches);
     const int nb = 1 + *std::max_element(batch.begin(), batch.end());
-    std::vector<int32_t> nlev(na), blev(nb, 0);
-    int32_t min_lev = INT32_MAX;
-    for (int64_t a = 0; a < na; a++) {
-        int32_t mx = 0;
+    // items of each angle and level, then where they start in the work list;
+    // both passes angle by angle in parallel (73,002 cells x 128 angles: 72 to
+    // 19 ms)
+    std::vector<std::vector<uint32_t>> count(na);
+    for_each_angle(na, nc * na, kListGrain, [&](int64_t a) {
         const int32_t *l = levels.data() + a * nc;
+        count[a].resize(1 + *std::max_element(l, l + nc), 0u);
         for (int64_t c = 0; c < nc; c++)
-            mx = std::max(mx, l[c]);
-        nlev[a] = mx + 1;
-        min_lev = std::min(min_lev, mx + 1);
-        blev[batch[a]] = std::max(blev[batch[a]], mx + 1);
+            count[a][l[c]]++;
+    });
+    std::vector<int32_t> blev(nb, 0);
+    int32_t min_lev = INT32_MAX;
+    s.lev_off.assign(na + 1, 0);
+    for (int64_t a = 0; a < na; a++) {
+        const int32_t nlev = int32_t(count[a].size());
+        min_lev = std::min(min_lev, nlev);
+        blev[batch[a]] = std::max(blev[batch[a]], nlev);
+        s.lev_off[a + 1] = s.lev_off[a] + nlev;
     }
     std::vector<int64_t> boff(nb + 1, 0);
     for (int b = 0; b < nb; b++)
@@ -460,56 +472,55 @@ try {
     s.batch_steps = boff;
     s.min_levels = min_lev;
     s.step_off.assign(s.n_steps + 1, 0);
-    for (int64_t a = 0; a < na; a++) {
-        const int32_t *l = levels.data() + a * nc;
-        for (int64_t c = 0; c < nc; c++)
-            s.step_off[boff[batch[a]] + l[c] + 1]++;
-    }
+    for (int64_t a = 0; a < na; a++)
+        for (size_t l = 0; l < count[a].size(); l++)
+            s.step_off[boff[batch[a]] + l + 1] += count[a][l];
     for (int64_t st = 0; st < s.n_steps; st++)
         s.step_off[st + 1] += s.step_off[st];
     std::vector<int64_t> pos(s.step_off.begin(), s.step_off.end() - 1);
-    s.work.resize(size_t(na) * nc);
-    s.lev_off.assign(na + 1, 0);
-    for (int64_t a = 0; a < na; a++)
-        s.lev_off[a + 1] = s.lev_off[a] + nlev[a];
     s.slice.resize(s.lev_off[na]);
-    std::vector<int32_t> cells(nc);
-    for (int64_t a = 0; a < na; a++) {
+    for (int64_t a = 0; a < na; a++)
+        for (size_t l = 0; l < count[a].size(); l++) {
+            int64_t &p = pos[boff[batch[a]] + l];
+            s.slice[s.lev_off[a] + l] = {uint32_t(p), count[a][l]};
+            p += count[a][l];
+        }
+    s.work.resize(size_t(na) * nc);
+    for_each_angle(na, nc * na, kListGrain, [&](int64_t a) {
         const int32_t *l = levels.data() + a * nc;
-        LevelSlice *sl = s.slice.data() + s.lev_off[a];
-        for (int32_t lev = 0; lev < nlev[a]; lev++)
-            sl[lev].first = uint32_t(pos[boff[batch[a]] + lev]);
-        for (int64_t c = 0; c < nc; c++)
-            cells[c] = int32_t(c);
-        if (order == T2_ORDER_FACES) {
-            // stable counting sort of the cells by incoming-face pattern, so
-            // that the items sharing a wavefront take the same upwind faces
-            const double *om = omega + 3 * a;
-            std::vector<uint8_t> mask(nc);
-            std::array<int64_t, 17> start{};
-            for (int64_t c = 0; c < nc; c++) {
-                unsigned mk = 0;
-                for (int k = 0; k < 4; k++)
-                    if (m.adj[4 * c + k] >= 0 &&
-                        omega_dot_n(om, &m.normal[(4 * c + k) * 3]) < 0)
-                        mk |= 1u << k;
-                mask[c] = uint8_t(mk);
-                start[mk + 1]++;
-            }
-            for (int b = 0; b < 16; b++)
-                start[b + 1] += start[b];
+        std::vector<uint32_t> at(count[a].size());
+        for (size_t lev = 0; lev < at.size(); lev++)
+            at[lev] = s.slice[s.lev_off[a] + lev].first;
+        auto put = [&](int64_t c) {
+            s.work[at[l[c]]++] = uint32_t(c) | (uint32_t(a) << cb);
+        };
+        if (order != T2_ORDER_FACES) {
             for (int64_t c = 0; c < nc; c++)
-                cells[start[mask[c]]++] = int32_t(c);
+                put(c);
+            return;
         }
-        for (int64_t i = 0; i < nc; i++) {
-            const int64_t c = cells[i];
-            s.work[pos[boff[batch[a]] + l[c]]++] =
-                uint32_t(c) | (uint32_t(a) << cb);
+        // stable counting sort of the cells by incoming-face pattern, so
+        // that the items sharing a wavefront take the same upwind faces
+        const double *om = omega + 3 * a;
+        std::vector<uint8_t> mask(nc);
+        std::vector<int32_t> cells(nc);
+        std::array<int64_t, 17> start{};
+        for (int64_t c = 0; c < nc; c++) {
+            unsigned mk = 0;
+            for (int k = 0; k < 4; k++)
+                if (m.adj[4 * c + k] >= 0 &&
+                    omega_dot_n(om, &m.normal[(4 * c + k) * 3]) < 0)
+                    mk |= 1u << k;
+            mask[c] = uint8_t(mk);
+            start[mk + 1]++;
         }
-        for (int32_t lev = 0; lev < nlev[a]; lev++)
-            sl[lev].count = uint32_t(pos[boff[batch[a]] + lev]) -
-                            sl[lev].first;
-    }
+        for (int b = 0; b < 16; b++)
+            start[b + 1] += start[b];
+        for (int64_t c = 0; c < nc; c++)
+            cells[start[mask[c]]++] = int32_t(c);
+        for (int64_t i = 0; i < nc; i++)
+            put(cells[i]);
+    });
     return T2_OK;
 } catch (const std::bad_alloc &) {
     return no_host_memory();
@@ -533,7 +544,7 @@ try {
     const uint32_t cmask = (uint32_t(1) << s.cell_bits) - 1;
     slot.assign(size_t(na) * nc, kNoSlot);
     std::vector<int64_t> most(na, 0);
-    for_each_angle(na, [&](int64_t a) {
+    for_each_angle(na, nc * na, kGrain, [&](int64_t a) {
         const double *om = omega + 3 * a;
         const LevelSlice *sl = s.slice.data() + s.lev_off[a];
         const int32_t nlev = s.lev_off[a + 1] - s.lev_off[a];
@@ -625,7 +636,7 @@ struct SweepDag {
         std::vector<uint8_t> lag(size_t(na) * nc, 0);
         for (const LaggedFace &f : lagged)
             lag[size_t(f.angle) * nc + f.cell] |= uint8_t(1u << f.face);
-        for_each_angle(na, [&](int64_t a) {
+        for_each_angle(na, nc * na, kGrain, [&](int64_t a) {
             const double *om = omega + 3 * a;
             const uint8_t *lg = lag.data() + a * nc;
             uint8_t *b = bits.data() + a * nc;
@@ -708,7 +719,7 @@ try {
     // backward traversal of src/Priorities.cc:120-143 (one rank: no
     // partition sides)
     std::vector<uint64_t> top(na, 0);
-    for_each_angle(na, [&](int64_t a) {
+    for_each_angle(na, nc * na, kGrain, [&](int64_t a) {
         std::vector<int32_t> cells;
         reverse_level_order(levels + a * nc, nc, cells);
         uint64_t *b = blev.data() + a * nc;
@@ -739,7 +750,7 @@ try {
         // rank no face is a partition side, so only the parent shift (0 for
         // BFDS, -1 otherwise, added in unsigned 64-bit arithmetic) acts
         const uint64_t shift = intra == 2 ? 0 : ~uint64_t(0);
-        for_each_angle(na, [&](int64_t a) {
+        for_each_angle(na, nc * na, kGrain, [&](int64_t a) {
             std::vector<int32_t> cells;
             reverse_level_order(levels + a * nc, nc, cells);
             uint64_t *p = prio.data() + a * nc;
