@@ -365,13 +365,19 @@ int ensure_stall_flag(StallFlag *f)
 {
     if (f->host)
         return T2_OK;
-    int32_t *h = nullptr;
-    T2_HIP(hipHostMalloc(reinterpret_cast<void **>(&h), sizeof(int32_t),
-                         hipHostMallocMapped | hipHostMallocCoherent));
-    *h = 0;
-    f->host = h;
-    T2_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&f->device), h,
-                                   0));
+    void *h = nullptr, *d = nullptr;
+    if (hipHostMalloc(&h, sizeof(int32_t),
+                      hipHostMallocMapped | hipHostMallocCoherent) !=
+            hipSuccess ||
+        hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        if (h)
+            (void)hipHostFree(h);
+        return fail(T2_ERR_NOMEM, "pinned host memory for a sweep's flag");
+    }
+    f->host = static_cast<int32_t *>(h);
+    f->device = static_cast<int32_t *>(d);
+    *f->host = 0;
     return T2_OK;
 }
 
