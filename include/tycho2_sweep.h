@@ -65,7 +65,7 @@ typedef struct t2_sweeper t2_sweeper;
 
 typedef struct {
     int64_t n_cells, n_angles, n_groups;
-    int64_t n_steps;          /* sweep steps (max levels over angles)      */
+    int64_t n_steps;          /* schedule steps (max levels over angles)   */
     int64_t min_levels;       /* fewest levels of any angle                */
     int64_t n_lagged;         /* (angle, cell, face) triples lagged        */
     int64_t psi_bytes;        /* device bytes of the angular flux          */
@@ -103,7 +103,9 @@ int t2_mesh_geometry(int64_t n_cells, int64_t n_nodes, const double *coords,
  * (replaces GraphTraverser's ready queue, src/GraphTraverser.cc:467-644).
  * Dependency cycles, on which the reference's traversal never ends, are
  * broken by lagging the weakest unmet face (smallest A |Omega.n|); the number
- * of lagged (angle, cell, face) triples is returned in *n_lagged. */
+ * of lagged (angle, cell, face) triples is returned in *n_lagged.  (A handle's
+ * schedule levels an angle with lagged faces again without them, in fewer
+ * levels: t2_info.n_steps.) */
 int t2_sweep_levels(int64_t n_cells, const int64_t *adj_cell,
                     const double *area, const double *normal,
                     int64_t n_angles, const double *omega, int32_t *levels,
@@ -311,8 +313,8 @@ int t2_solve_source_iteration(t2_sweeper *s, int64_t iter_max, double err_max,
  * process ends) instead of the handle's buffers, and the call makes no
  * allocation, graph instantiation or stream creation: a sweep whose hipGraph
  * is not captured yet is launched step by step.  The array's size does not
- * depend on the problem (the reduction runs 1024 blocks over any length),
- * so no problem size exceeds it.  Returns T2_ERR_STATE when a resource
+ * depend on the problem (the reduction runs at most 1024 blocks over any
+ * length), so no problem size exceeds it.  Returns T2_ERR_STATE when a resource
  * would have to be created first: the ready-queue tables of
  * T2_ENGINE_QUEUE / T2_ENGINE_HYBRID and the streams of concurrent angle
  * batches are made by the handle's first ordinary sweep or solve.  Every

@@ -995,7 +995,8 @@ void free_angle_form(t2_sweeper *s)
 // kMinAngleBlocks blocks, because a block's records are read once per gc
 // groups.  256, 128 and 64 blocks, us: 24,576 cells x 32 angles x 16 groups
 // FP64 a sweep alone 335, 398, 843, a pass among three handles 417, 326, 496;
-// 6,000 x 32 x 16 87, 93, 131 and 114, 79, 79.
+// 6,000 x 32 x 16 87, 93, 131 and 114, 79, 79: 128 lose 7 to 19% alone and
+// gain 22 to 31% among three.
 constexpr int64_t kMinAngleBlocks = 128;
 
 int angle_groups(const t2_sweeper *s, int64_t slots)
@@ -1029,7 +1030,8 @@ int angle_groups(const t2_sweeper *s, int64_t slots)
 //   73,002        128         16        FP64  3684 /  3930    5921 / 3757 *
 //   82,944        128         32        FP32  4385 /  4615    6944 / 4463 *
 //  131,712        128          4        FP64  2318 /  2777    2962 / 2153 *
-// (* not taken).
+// (* not taken: that costs 5 to 20% alone and saves 27 to 37% among three).
+// t2_set_form has the step launches where the rule is wrong for a caller.
 bool angle_pays(const t2_sweeper *s, int gc)
 {
     if (gc <= 0)

@@ -1013,12 +1013,12 @@ buffer_store_piece(Rsrc r, uint32_t off, const X *x,
 // or four vertices of a cell leave in one access; and the next round's loads
 // go before the stores, without a branch between them, so that waiting for
 // them does not wait for the stores.  A sweep of 34,992 cells x 128 angles x 4
-// groups FP64: 533 -> 409 us, 2.2 TB/s of its 0.92 GB (252 us without stores,
-// 342 without loads, no less without the waits between levels);
-// 48,000 x 288 x 8 FP32: 1860 -> 1300 us; 24,576 x 32 x 16 FP64, whose rows
-// are lines: 419 -> 403.  Small problems are bound by the levels: 0.5 to
-// 0.6 us each (750 x 32 x 1 FP64 in 24 us, 6,000 x 32 x 4 in 62; step launches
-// take 3.6 us a level).
+// groups FP64: 533 -> 409 us (378 under a trace: 2.5 TB/s of its 0.94 GB; of
+// the 533, 252 are left without stores, 342 without loads, no less without the
+// waits between levels); 48,000 x 288 x 8 FP32: 1860 -> 1300 us; 24,576 x 32 x
+// 16 FP64, whose rows are lines: 419 -> 403.  Small problems are bound by the
+// levels: 0.45 to 0.55 us each (750 x 32 x 1 FP64 in 22 us, 6,000 x 32 x 4 in
+// 57; step launches take 3.6 us a level).
 //
 // ANG: angle-dependent source, 0 none, 1 FP64 (src_ang), 2 T (src_ang_t).
 // ROW: one group in all, so that a cell's four values are contiguous and move
@@ -1891,8 +1891,9 @@ struct alignas(16) Vec16 {
 
 // phi = sum_a w_a psi_a; kMomentMinus: phi = x - sum_a w_a psi_a (the Krylov
 // operator); kMomentL1: the partial sums of |phi - x| and |phi| as well (the
-// change of a source-iteration step).  Bound by reading psi, 5 to 5.5 TB/s
-// (34,992 cells x 128 angles x 4 groups FP64 in 115 us); at small sizes by its
+// change of a source-iteration step).  Bound by reading psi, 4.7 TB/s of 34,992
+// cells x 128 angles x 4 groups FP64 (122 us) to 5.5 TB/s of 384,000 x 128 x
+// 16; at small sizes by its
 // launch, so what follows it on phi is done here: 21 steps of source iteration
 // on 750 x 32 x 1 FP64 1300 -> 1240 us.
 enum MomentMode { kMoment = 0, kMomentMinus = 1, kMomentL1 = 2 };
