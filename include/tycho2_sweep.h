@@ -172,16 +172,17 @@ int t2_sweeper_info(const t2_sweeper *s, t2_info *info);
 
 /* Launch shape of the step launches and the ready queue: cells per block and
  * groups per lane (autotuner knobs); 0 keeps what is set.  A number of cells
- * per block also sets T2_FORM_STEPS. */
+ * per block also selects T2_FORM_STEPS (the one launch's tables stay). */
 int t2_set_launch(t2_sweeper *s, int items_per_block, int groups_per_lane);
 
 /* Form of the level engine's sweeps.  T2_FORM_AUTO (default): small and deep
  * problems in one launch, a block sweeping an angle through its levels, while
  * the knobs of the step launches (groups and items per lane, angle batches)
- * are at their defaults; T2_FORM_STEPS: one launch per schedule step whatever
- * the problem.  Results are bitwise the same.  Where the device has no memory
- * for the one launch's tables, or a later call needs theirs, the handle makes
- * step launches until its schedule is next rebuilt. */
+ * are at their defaults.  T2_FORM_STEPS: one launch per schedule step whatever
+ * the problem; the device memory of the one launch's tables is given back, and
+ * T2_FORM_AUTO builds the schedule anew for them.  Results are bitwise the
+ * same.  Where the device has no memory for the tables, or a later call needs
+ * theirs, the handle makes step launches until its schedule is next built. */
 #define T2_FORM_AUTO 0
 #define T2_FORM_STEPS 1
 int t2_set_form(t2_sweeper *s, int form);

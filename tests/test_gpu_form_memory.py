@@ -120,3 +120,27 @@ def test_member_of_a_batch_makes_room(precision):
         b.synchronize()
     for m in mem:
         m.close()
+
+
+def test_steps_give_the_tables_back():
+    print("form tables given back", flush=True)
+    with handle(5, 4, 4, FP64) as s:
+        s.sweep_step()
+        ref, full = s.phi(), s.info()["device_bytes"]
+        items = s.nc * s.na
+        for _ in range(2):
+            s.set_form(FORM_STEPS)
+            assert s.form() == 0
+            assert s.info()["device_bytes"] <= full - 32 * items
+            s.set_order(0)                       # none built either
+            s.set_order(1)
+            assert s.info()["device_bytes"] <= full - 32 * items
+            s.set_phi(np.zeros_like(ref))
+            s.sweep_step()
+            assert np.array_equal(s.phi(), ref)
+            s.set_form(0)
+            assert s.form() > 0
+            assert s.info()["device_bytes"] == full
+            s.set_phi(np.zeros_like(ref))
+            s.sweep_step()
+            assert np.array_equal(s.phi(), ref)

@@ -79,6 +79,7 @@ struct t2_sweeper {
     int block = 256, gpl = 1, batches = 1, order = T2_ORDER_FACES;
     int ipl = 1;                     // items per lane (level engine)
     int form = T2_FORM_AUTO;         // of the level engine's sweeps
+    bool no_tables = false;          // T2_FORM_STEPS left the tables out
     int intra = -1, inter = 0;       // priority schedule (intra < 0: levels)
     int64_t step_width = 0;
     double dep_tol = t2::kTraverseRule;   // dependency rule of the schedule
@@ -1103,7 +1104,8 @@ try {
 void start_angle_tables(t2_sweeper *s)
 {
     const auto &sc = s->sched;
-    if (sc.slice.empty() || s->batches != 1 || !s->use_graph ||
+    s->no_tables = s->form == T2_FORM_STEPS;
+    if (s->no_tables || sc.slice.empty() || s->batches != 1 || !s->use_graph ||
         s->gauss != T2_GAUSS_NOPIVOT ||
         s->n_phi() * int64_t(sizeof(double)) >= (int64_t(1) << 32))
         return;
@@ -1801,6 +1803,14 @@ int t2_set_form(t2_sweeper *s, int form)
     if (form != T2_FORM_AUTO && form != T2_FORM_STEPS)
         return fail(T2_ERR_ARG, "form must be T2_FORM_AUTO or T2_FORM_STEPS");
     s->form = form;
+    if (form == T2_FORM_STEPS ? s->angle_gc == 0 : !s->no_tables)
+        return T2_OK;
+    T2_TRY(set_device(s));
+    T2_HIP(hipStreamSynchronize(s->stream));
+    if (form == T2_FORM_AUTO)
+        return build_schedule_device(s);
+    free_angle_form(s);
+    s->no_tables = true;
     return T2_OK;
 }
 
