@@ -1249,9 +1249,12 @@ __device__ __forceinline__ void sweep_angle(const SweepArgs<T> &p,
         r2 = round_at(k + 3 * n_waves);
 
         compute_here(f);
+        // (FP32's are two instructions each; held from here they cost 384,000
+        // cells x 32 angles x 2 groups 0.8%)
+        if constexpr (!kEarly)
 #pragma unroll
-        for (int i = 0; i < 12; i++)
-            compute_here(at[i]);
+            for (int i = 0; i < 12; i++)
+                compute_here(at[i]);
 
         auto ready = [&]() {
             return __builtin_amdgcn_readfirstlane(__hip_atomic_load(
